@@ -1,0 +1,405 @@
+// Attention on the matrix cores in fp32: out = softmax(q k^T * scale) v for
+// grouped-query heads, over all keys or causal, with an online softmax.
+//
+// The scores and the weighted sum are contractions, so they run on
+// v_mfma_f32_32x32x2_f32: fp32 operands, products and sums, as the VALU loops
+// this replaces (same inf / NaN behaviour), at twice the VALU's rate. Both are
+// formed transposed: S^T = K Q^T and O^T = V^T P^T. A column of either is one
+// (query, head) pair, held by lanes c and c + 32, so
+//   - the softmax of a column is arithmetic inside a lane plus one exchange
+//     between the two halves, and rescaling O^T is a multiply per register;
+//   - accumulator register e of S^T (keys 8 (e / 4) + 4 h + e % 4 of the tile
+//     for half h) is, after the exp, the B operand of step e of O^T: the keys of
+//     that step are the ones the two halves hold, and V's rows are loaded to
+//     match. The probabilities never leave their registers.
+// The G query heads of a kv head are columns of the same tile, so K and V are
+// read once for all of them.
+//
+// A workgroup owns 32 columns; its 4 waves take every 4th tile of 32 keys,
+// loaded straight into registers in operand layout (32 KB of K and V per tile
+// for 128 MFMAs of 64 cycles: 4 B per cycle and wave, far below what L2
+// serves, so sharing tiles through LDS would buy nothing), the next K tile in
+// flight during V's product, V during K's and the softmax, each in halves (all
+// of both in flight spilled registers: 88 us against 72 in the first case
+// below). The columns' q is in LDS. The waves' (max, sum, O) meet in LDS at
+// the end. When there are too few column tiles
+// for the CUs (decode steps: B * Hk tiles), the keys are split over workgroups
+// as well and a second launch merges the partials; such a launch is bound by
+// reading K and V, and the idle columns of its MFMAs cost no time.
+//
+// Measured (MI355X; before: a workgroup per query row on the VALU, keys one by
+// one): 777 queries and keys, 16 heads over 8, D 128: 909 -> 72 us; one query
+// of 4 sequences over 2047 keys: 578 -> 27 us (2.5 TB/s); causal over 1021
+// positions: 462 -> 57 us. Bound by the fp32 MFMA (35 us of it in the first)
+// and by the softmax between its two products, which two waves per SIMD only
+// partly cover. Error against 64 bits 3.1e-7 (was 5.2e-7) and 2.3e-7 (8.2e-7).
+#include "attention.hpp"
+
+#include <algorithm>
+#include <float.h>
+
+namespace pio {
+
+typedef float at_f4 __attribute__((ext_vector_type(4)));
+typedef float at_f2 __attribute__((ext_vector_type(2)));
+typedef float at_v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 at_h4 __attribute__((ext_vector_type(4)));
+typedef _Float16 at_h8 __attribute__((ext_vector_type(8)));
+
+constexpr int AT_COLS = 32;    // (query, head) pairs per workgroup
+constexpr int AT_KEYS = 32;    // keys per tile
+constexpr int AT_WAVES = 4;
+
+struct AttnParams {
+    AttnArgs a;
+    int G, tiles;              // query heads per kv head; column tiles per (b, kv head)
+    int splits, per_split;     // key tiles per split (a multiple of AT_WAVES)
+    float* part_o;             // [splits][B * Hk * tiles * 32][D] when splits > 1
+    float* part_ml;            // [splits][..][2]
+};
+
+template <int D>
+constexpr size_t at_lds_bytes() { return (size_t)AT_WAVES * AT_COLS * (D + 4) * 4; }
+
+// Vector types of a lane's loads: 16 bytes of a K row, D / 32 elements of a V row.
+template <typename KT, int D> struct AtRaw;
+template <> struct AtRaw<float, 128> { typedef at_f4 k, v; };
+template <> struct AtRaw<float, 64> { typedef at_f4 k; typedef at_f2 v; };
+template <> struct AtRaw<_Float16, 128> { typedef at_h8 k; typedef at_h4 v; };
+
+// Dimension held by slot sl of a row (fp16 cache rows pair dims i and i + 64).
+template <bool PAIR>
+__device__ __forceinline__ int at_dim(int sl) { return PAIR ? (sl >> 1) + 64 * (sl & 1) : sl; }
+
+// Slot of the first of the 4 steps in K group c of half h: a lane's 16-byte
+// load covers one group of fp32 or two of fp16.
+template <typename KT>
+__device__ __forceinline__ int at_slot(int c, int h) {
+    return sizeof(KT) == 4 ? 8 * c + 4 * h : 16 * (c >> 1) + 8 * h + 4 * (c & 1);
+}
+
+template <int D, typename KT, bool CAUSAL>
+__global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams p) {
+    constexpr bool PAIR = sizeof(KT) == 2;
+    constexpr int NT = D / 32;             // O^T tiles: row i of tile n is slot NT * i + n
+    constexpr int NC = D / 8;              // K groups of 4 steps
+    constexpr int OP = D + 4;              // LDS pitch of the merge (floats)
+    extern __shared__ __attribute__((aligned(16))) float at_lds[];
+    __shared__ float at_m[AT_WAVES][AT_COLS], at_l[AT_WAVES][AT_COLS];
+    const AttnArgs& a = p.a;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int col = lane & 31, h = lane >> 5;
+
+    // kv heads fastest: with 8 of them each XCD's L2 holds one head's K and V
+    int x = blockIdx.x;
+    const int g = x % a.Hk;
+    x /= a.Hk;
+    const int b = x % a.B;
+    int ct = x / a.B;
+    if (CAUSAL) {
+        // Later tiles see more keys. In dispatch order the first 256 workgroups
+        // (one per CU) take tiles from the long end, the next 256 from the
+        // short end, and so on, so that a CU's two have about the same sum.
+        const int run = max(1, 256 / (a.B * a.Hk)), n = ct / run, r = (n >> 1) * run + ct - n * run;
+        ct = n & 1 ? r : p.tiles - 1 - r;
+    }
+    const int ncols = a.S * p.G, c0 = ct * AT_COLS;
+    const int last_s = (min(c0 + AT_COLS, ncols) - 1) / p.G;
+    const int limit_all = CAUSAL ? a.pos0 + last_s + 1 : a.T;       // keys any column sees
+    const int tiles_all = (limit_all + AT_KEYS - 1) / AT_KEYS;
+    const int kt0 = blockIdx.y * p.per_split, kt1 = min(kt0 + p.per_split, tiles_all);
+
+    // q of the columns -> LDS, in the order the S^T steps read it
+    for (int i = tid; i < AT_COLS * (D / 4); i += 64 * AT_WAVES) {
+        const int c = i / (D / 4), grp = i % (D / 4);              // group grp = 2 c4 + half
+        const int cc = min(c0 + c, ncols - 1), s = cc / p.G, hd = g * p.G + cc - s * p.G;
+        const float* qr = a.q + b * a.q_b + (int64_t)s * a.q_s + hd * D;
+        const int sl = at_slot<KT>(grp >> 1, grp & 1);
+        at_f4 v;
+        if constexpr (PAIR) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = qr[at_dim<PAIR>(sl + e)];
+        } else {
+            v = *(const at_f4*)(qr + sl);
+        }
+        *(at_f4*)(at_lds + (grp * AT_COLS + c) * 4) = v;
+    }
+    __syncthreads();
+
+    const KT* kb = (const KT*)a.k + b * a.kv_b + g * a.kv_h;
+    const KT* vb = (const KT*)a.v + b * a.kv_b + g * a.kv_h;
+    const int mycol = min(c0 + col, ncols - 1);
+    const int limit = CAUSAL ? a.pos0 + mycol / p.G + 1 : a.T;
+
+    at_v16f o[NT];
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) o[n][e] = 0.f;
+    float m = a.m_seed, l = 0.f;
+
+    // A tile's K: 4 steps per group from the row of this lane's key; its V: the
+    // rows of the 16 steps' keys, NT consecutive slots per lane. Raw bits, so
+    // that fp16 is widened at its use and the loads stay in flight together.
+    // Rows past the last key re-read it (their weights and V are zeroed below).
+    typedef typename AtRaw<KT, D>::k at_kt;
+    typedef typename AtRaw<KT, D>::v at_vt;
+    constexpr int KL = D * (int)sizeof(KT) / 32;     // K loads of 16 bytes
+    at_kt kr[KL];
+    at_vt vr[16];
+    const int k_lane = col * a.kv_t + h * (16 / (int)sizeof(KT));
+    const int v_lane = 4 * h * a.kv_t + NT * col;
+    auto load_k = [&](int kt, int half) {
+        const int t0 = kt * AT_KEYS;
+        const KT* r = t0 + AT_KEYS <= limit_all
+                          ? kb + (int64_t)t0 * a.kv_t + k_lane
+                          : kb + (int64_t)min(t0 + col, limit_all - 1) * a.kv_t + h * (16 / (int)sizeof(KT));
+#pragma unroll
+        for (int c = half * (KL / 2); c < (half + 1) * (KL / 2); c++)
+            kr[c] = *(const at_kt*)(r + c * (32 / (int)sizeof(KT)));
+    };
+    auto load_v = [&](int kt, int half) {
+        const int t0 = kt * AT_KEYS;
+        if (t0 + AT_KEYS <= limit_all) {
+            const KT* tb = vb + (int64_t)t0 * a.kv_t;
+#pragma unroll
+            for (int e = 8 * half; e < 8 * half + 8; e++)
+                vr[e] = *(const at_vt*)(tb + (8 * (e >> 2) + (e & 3)) * a.kv_t + v_lane);
+        } else {
+#pragma unroll
+            for (int e = 8 * half; e < 8 * half + 8; e++) {
+                const int t = min(t0 + 8 * (e >> 2) + 4 * h + (e & 3), limit_all - 1);
+                vr[e] = *(const at_vt*)(vb + (int64_t)t * a.kv_t + NT * col);
+            }
+        }
+    };
+    auto k_at = [&](int c, int e) {
+        if constexpr (PAIR) return (float)kr[c >> 1][4 * (c & 1) + e];
+        else return (float)kr[c][e];
+    };
+
+    int kt = kt0 + w;
+    if (kt < kt1) {
+        load_k(kt, 0);
+        load_k(kt, 1);
+    }
+    for (; kt < kt1; kt += AT_WAVES) {
+        load_v(kt, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        // scores as 4 chains of D / 4 terms, added: half the rounding of one
+        // chain, whose error is the larger part of the probabilities'
+        at_v16f s;
+#pragma unroll
+        for (int ch = 0; ch < 4; ch++) {
+            at_v16f t;
+#pragma unroll
+            for (int e = 0; e < 16; e++) t[e] = 0.f;
+#pragma unroll
+            for (int c = ch * (NC / 4); c < (ch + 1) * (NC / 4); c++) {
+                const at_f4 qv = *(const at_f4*)(at_lds + ((2 * c + h) * AT_COLS + col) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) t = __builtin_amdgcn_mfma_f32_32x32x2f32(k_at(c, e), qv[e], t, 0, 0, 0);
+            }
+            if (ch == 0) s = t;
+            else s += t;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(kt, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const int t0 = kt * AT_KEYS;
+        const bool more = kt + AT_WAVES < kt1;
+        // wave-uniform: some key of the tile is past some column's last one
+        const bool edge = t0 + AT_KEYS > (CAUSAL ? a.pos0 + c0 / p.G + 1 : a.T);
+        float mt = m;
+#pragma unroll
+        for (int e = 0; e < 16; e++) s[e] *= a.scale;
+        if (edge) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const int t = t0 + 8 * (e >> 2) + 4 * h + (e & 3);
+                if (t < limit) mt = fmaxf(mt, s[e]);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 16; e++) mt = fmaxf(mt, s[e]);
+        }
+        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+        const float corr = expf(m - mt);
+        float sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            s[e] = expf(s[e] - mt);
+            if (edge && t0 + 8 * (e >> 2) + 4 * h + (e & 3) >= limit) s[e] = 0.f;
+            sum += s[e];
+        }
+        l = l * corr + sum;
+        if (__any(mt != m)) {
+#pragma unroll
+            for (int n = 0; n < NT; n++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) o[n][e] *= corr;
+        }
+        m = mt;
+        // a key past the last one: its weight is zero, and what is read in its
+        // place must not be inf or NaN. (A causal tile's later keys are rows of
+        // this batch: an inf there also meets zero weights of earlier columns.)
+        auto zero_v = [&](int e) {
+            if (edge && t0 + 8 * (e >> 2) + 4 * h + (e & 3) >= limit_all)
+#pragma unroll
+                for (int n = 0; n < NT; n++) vr[e][n] = 0;
+        };
+#pragma unroll
+        for (int e = 0; e < 8; e++) zero_v(e);
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+#pragma unroll
+            for (int n = 0; n < NT; n++) o[n] = __builtin_amdgcn_mfma_f32_32x32x2f32((float)vr[e][n], s[e], o[n], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) load_k(kt + AT_WAVES, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 8; e < 16; e++) zero_v(e);
+#pragma unroll
+        for (int e = 8; e < 16; e++)
+#pragma unroll
+            for (int n = 0; n < NT; n++) o[n] = __builtin_amdgcn_mfma_f32_32x32x2f32((float)vr[e][n], s[e], o[n], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) load_k(kt + AT_WAVES, 1);
+    }
+
+    // the waves' columns meet in LDS: common maximum, scaled sums
+    l += __shfl_xor(l, 32, 64);
+    if (h == 0) {
+        at_m[w][col] = m;
+        at_l[w][col] = l;
+    }
+    __syncthreads();   // and every wave is done with q
+    float mx = at_m[0][col];
+#pragma unroll
+    for (int i = 1; i < AT_WAVES; i++) mx = fmaxf(mx, at_m[i][col]);
+    const float f = expf(m - mx);
+    float* ob = at_lds + (w * AT_COLS + col) * OP;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const int i = 8 * (e >> 2) + 4 * h + (e & 3);
+#pragma unroll
+        for (int n = 0; n < NT; n++) ob[NT * i + n] = o[n][e] * f;
+    }
+    __syncthreads();
+    for (int i = tid; i < AT_COLS * (D / 4); i += 64 * AT_WAVES) {
+        const int c = i / (D / 4), sl = (i % (D / 4)) * 4;
+        if (c0 + c >= ncols) continue;
+        at_f4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < AT_WAVES; k++) v += *(const at_f4*)(at_lds + (k * AT_COLS + c) * OP + sl);
+        float cm = at_m[0][c], cl = 0.f;
+#pragma unroll
+        for (int k = 1; k < AT_WAVES; k++) cm = fmaxf(cm, at_m[k][c]);
+#pragma unroll
+        for (int k = 0; k < AT_WAVES; k++) cl += at_l[k][c] * expf(at_m[k][c] - cm);
+        if (p.splits > 1) {
+            const int64_t row = ((int64_t)blockIdx.y * a.B + b) * a.Hk + g;
+            const int64_t at = row * p.tiles * AT_COLS + c0 + c;
+            *(at_f4*)(p.part_o + at * D + sl) = v;
+            if (sl == 0) {
+                p.part_ml[2 * at] = cm;
+                p.part_ml[2 * at + 1] = cl;
+            }
+            continue;
+        }
+        const float inv = 1.0f / cl;
+        const int s = (c0 + c) / p.G, hd = g * p.G + (c0 + c) - s * p.G;
+        float* orow = a.out + b * a.o_b + (int64_t)s * a.o_s + hd * D;
+        if constexpr (PAIR) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) orow[at_dim<PAIR>(sl + e)] = v[e] * inv;
+        } else {
+            *(at_f4*)(orow + sl) = v * inv;
+        }
+    }
+}
+
+// One column per D / 4 threads: the key splits' (max, sum, O) merged, in split order.
+template <int D, bool PAIR>
+__global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
+    constexpr int TPC = D / 4;
+    const AttnArgs& a = p.a;
+    const int ncols = a.S * p.G;
+    const int64_t i = (int64_t)blockIdx.x * (256 / TPC) + threadIdx.x / TPC;   // (b, kv head, column)
+    if (i >= (int64_t)a.B * a.Hk * ncols) return;
+    const int sl = (threadIdx.x % TPC) * 4;
+    const int64_t bg = i / ncols;
+    const int c = (int)(i - bg * ncols), b = (int)(bg / a.Hk), g = (int)(bg - (int64_t)b * a.Hk);
+    const int64_t step = (int64_t)a.B * a.Hk * p.tiles * AT_COLS, at = bg * p.tiles * AT_COLS + c;
+    float mx = p.part_ml[2 * at];
+#pragma unroll 8
+    for (int z = 1; z < p.splits; z++) mx = fmaxf(mx, p.part_ml[2 * (at + z * step)]);
+    float l = 0.f;
+    at_f4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int z = 0; z < p.splits; z++) {
+        const float f = expf(p.part_ml[2 * (at + z * step)] - mx);
+        l += p.part_ml[2 * (at + z * step) + 1] * f;
+        v += *(const at_f4*)(p.part_o + (at + z * step) * D + sl) * f;
+    }
+    const float inv = 1.0f / l;
+    const int s = c / p.G, hd = g * p.G + c - s * p.G;
+    float* orow = a.out + b * a.o_b + (int64_t)s * a.o_s + hd * D;
+    if constexpr (PAIR) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) orow[at_dim<PAIR>(sl + e)] = v[e] * inv;
+    } else {
+        *(at_f4*)(orow + sl) = v * inv;
+    }
+}
+
+bool attn_mfma_supported(const AttnArgs& a) {
+    // causal: the decoder's cache (head_dim 128); fp16 keys only there
+    if (a.D != 128 && !(a.D == 64 && !a.causal)) return false;
+    if (a.kv16 && !a.causal) return false;
+    if (a.H % a.Hk || a.kv_t >= 1 << 25 || a.q_s % 4 || a.o_s % 4 || a.q_b % 4 || a.o_b % 4 || a.kv_t % 8 || a.kv_h % 8 || a.kv_b % 8)
+        return false;
+    return aligned16(a.q) && aligned16(a.k) && aligned16(a.v) && aligned16(a.out);
+}
+
+template <int D, typename KT, bool CAUSAL>
+static int attn_launch(AttnParams& p, hipStream_t st) {
+    const AttnArgs& a = p.a;
+    const size_t lds = at_lds_bytes<D>();
+    const dim3 grid((unsigned)((int64_t)p.tiles * a.B * a.Hk), p.splits);
+    PIO_TRY((allow_lds<attn_mfma_kernel<D, KT, CAUSAL>>(lds)));
+    attn_mfma_kernel<D, KT, CAUSAL><<<grid, 64 * AT_WAVES, lds, st>>>(p);
+    PIO_LAUNCHED();
+    if (p.splits > 1) {
+        const int64_t cols = (int64_t)a.B * a.Hk * a.S * p.G;
+        attn_merge_kernel<D, sizeof(KT) == 2><<<ceil_div(cols, 256 / (D / 4)), 256, 0, st>>>(p);
+        PIO_LAUNCHED();
+    }
+    return PIO_OK;
+}
+
+int attn_mfma(const AttnArgs& a, hipStream_t st) {
+    AttnParams p{};
+    p.a = a;
+    p.G = a.H / a.Hk;
+    const int64_t ncols = (int64_t)a.S * p.G;
+    p.tiles = ceil_div(ncols, AT_COLS);
+    const int64_t wgs = (int64_t)p.tiles * a.B * a.Hk;
+    // Key splits while the workgroups stay within two per CU (what the
+    // registers and LDS hold) and each keeps a tile for every wave.
+    const int kt = ceil_div(a.T, AT_KEYS);
+    int splits = (int)std::max<int64_t>(1, std::min<int64_t>(512 / std::max<int64_t>(wgs, 1), kt / AT_WAVES));
+    p.per_split = ceil_div(ceil_div(kt, splits), AT_WAVES) * AT_WAVES;
+    p.splits = ceil_div(kt, p.per_split);
+    Scratch ws;
+    if (p.splits > 1) {
+        const size_t cols = (size_t)p.splits * wgs * AT_COLS;
+        PIO_TRY(ws.get(cols * (a.D + 2) * sizeof(float), st));
+        p.part_o = (float*)ws.ptr;
+        p.part_ml = p.part_o + cols * a.D;
+    }
+    if (a.causal) return a.kv16 ? attn_launch<128, _Float16, true>(p, st) : attn_launch<128, float, true>(p, st);
+    return a.D == 128 ? attn_launch<128, float, false>(p, st) : attn_launch<64, float, false>(p, st);
+}
+
+}  // namespace pio

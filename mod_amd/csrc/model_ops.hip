@@ -8,7 +8,7 @@
 // shape from its own operand instead, and says so. fp32 device tensors only;
 // every op runs on the library's current stream and returns a status
 // (PIO_OK or a negative code with the message in tensor_last_error).
-#include "pio_common.hpp"
+#include "attention.hpp"
 
 #include <climits>
 
@@ -220,6 +220,9 @@ __global__ __launch_bounds__(MO_THREADS) void mo_embed_kernel(const float* __res
 }
 
 // ---------------------------------------------------------- attention ------
+// The general kernel: head sizes and addresses that attention.hip's
+// matrix-core kernel does not take (it wants head_dim 64 or 128 and 16-byte
+// aligned rows).
 // One block per (batch, query position, head): q [B, S, H, D], k / v
 // [B, T, Hk, D], out [B, S, H, D]. Scores q.k * scale over all T keys (no
 // mask, as the reference), softmax with max from -1e9 and the weights
@@ -470,6 +473,14 @@ PIO_EXPORT int tensor_scaled_dot_product_attention_status(Tensor* q, Tensor* k, 
     const int64_t blocks = (int64_t)B * S * H;
     PIO_REQUIRE(blocks <= INT_MAX, "tensor_scaled_dot_product_attention: too many query rows");
     if (blocks == 0 || D == 0) return PIO_OK;
+    AttnArgs at{};
+    at.q = q->data; at.k = k->data; at.v = v->data; at.out = out->data;
+    at.q_s = at.o_s = H * D; at.kv_t = Hk * D; at.kv_h = D;
+    at.q_b = at.o_b = (int64_t)S * H * D; at.kv_b = (int64_t)T * Hk * D;
+    at.B = B; at.S = S; at.T = T; at.H = H; at.Hk = Hk; at.D = D;
+    at.scale = scale;
+    at.m_seed = -1e9f;
+    if (attn_mfma_supported(at)) return attn_mfma(at, current_stream());
     const size_t lds = (size_t)T * sizeof(float);
     PIO_TRY(allow_lds<mo_sdpa_kernel>(lds));
     mo_sdpa_kernel<<<(unsigned)blocks, MO_THREADS, lds, current_stream()>>>(q->data, k->data, v->data, out->data, S, T,

@@ -119,6 +119,54 @@ def test_scaled_dot_product_attention(B, Bn, S, H, Hk, T, D):
     assert err <= RTOL, err
 
 
+@pytest.mark.parametrize("Bn,S,H,Hk,T,D", [
+    (1, 1, 2, 1, 1, 128),        # one column, one key
+    (2, 16, 16, 8, 33, 128),     # 32 columns per kv head: one full tile; one key past a key tile
+    (1, 17, 2, 2, 128, 64),      # a tile of 32 with 17 columns; one key tile per wave
+    (1, 11, 3, 1, 31, 128),      # 33 columns: the second tile holds one; a partial key tile
+    (1, 65, 4, 4, 65, 64), (3, 1, 16, 8, 1023, 128),   # keys split over workgroups, ragged last split
+    (1, 300, 8, 2, 517, 128), (2, 1, 32, 4, 4100, 64)])
+def test_attention_tiles(B, Bn, S, H, Hk, T, D):
+    """The matrix-core attention at the edges of its column and key tiles and of
+    its key splits, against the oracle and against the general kernel (which
+    takes the same operands at addresses that are not 16-byte aligned), out of
+    place and into q; a value row of inf in the last, partly filled key tile
+    reaches only its own dimension."""
+    from mod_amd import ops
+    from mod_amd.ops import lib
+    _say(f"attention tiles B{Bn} S{S} H{H} Hk{Hk} T{T} D{D}")
+    rng = np.random.default_rng(S * 7 + T)
+    q = rng.standard_normal((Bn, S, H, D)).astype(np.float32)
+    k = rng.standard_normal((Bn, T, Hk, D)).astype(np.float32)
+    v = rng.standard_normal((Bn, T, Hk, D)).astype(np.float32)
+    vmax = float(np.abs(v).max())
+    want = mo.sdpa(q, k, v, 1 / np.sqrt(D))
+    tq, tk, tv = _t(B, q), _t(B, k), _t(B, v)
+    got = B.scaled_dot_product_attention(tq, tk, tv).numpy()
+    assert float(np.abs(got - want).max()) <= RTOL * vmax
+
+    def shifted(a):      # the same tensor one float further on
+        own = B.Tensor([a.size + 1])
+        own.load(np.concatenate([[0.0], a.ravel()]).astype(np.float32))
+        c = own._handle.contents
+        shp = (ctypes.c_int * 4)(*a.shape)
+        ptr = ctypes.cast(ctypes.cast(c.data, ctypes.c_void_p).value + 4, ctypes.POINTER(ctypes.c_float))
+        return own, shp, ops.CTensor(ptr, ctypes.cast(shp, ctypes.POINTER(ctypes.c_int)), 4, a.size, c.device_id)
+
+    keep = [shifted(a) for a in (q, k, v, np.zeros_like(q))]
+    refs = [ctypes.byref(x[2]) for x in keep]
+    assert lib.tensor_scaled_dot_product_attention_status(*refs, ctypes.c_float(1 / np.sqrt(D))) == ops.OK
+    general = keep[3][0].numpy()[1:].reshape(q.shape)
+    assert float(np.abs(got - general).max()) <= RTOL * vmax
+    assert lib.tensor_scaled_dot_product_attention_status(tq._handle, tk._handle, tv._handle, tq._handle,
+                                                          ctypes.c_float(1 / np.sqrt(D))) == ops.OK
+    assert np.array_equal(tq.numpy(), got)
+    v[:, T - 1, :, 3] = np.inf
+    got = B.scaled_dot_product_attention(_t(B, q), tk, _t(B, v)).numpy()
+    assert np.all(got[..., 3] == np.inf)
+    assert np.isfinite(np.delete(got, 3, axis=-1)).all()
+
+
 def test_slice_set_slice_cat_reshape_exact(B):
     rng = np.random.default_rng(5)
     x = rng.standard_normal((3, 9, 4, 8)).astype(np.float32)
