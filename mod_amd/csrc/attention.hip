@@ -34,6 +34,7 @@
 // and by the softmax between its two products, which two waves per SIMD only
 // partly cover. Error against 64 bits 3.1e-7 (was 5.2e-7) and 2.3e-7 (8.2e-7).
 #include "attention.hpp"
+#include "wf_planes.hpp"
 
 #include <algorithm>
 #include <float.h>
@@ -76,6 +77,22 @@ __device__ __forceinline__ int at_dim(int sl) { return PAIR ? (sl >> 1) + 64 * (
 template <typename KT>
 __device__ __forceinline__ int at_slot(int c, int h) {
     return sizeof(KT) == 4 ? 8 * c + 4 * h : 16 * (c >> 1) + 8 * h + 4 * (c & 1);
+}
+
+// 4 consecutive slots from sl of (row s of batch b, query head hd).
+template <bool PAIR, bool CAUSAL>
+__device__ __forceinline__ void at_store(const AttnArgs& a, int D, int b, int s, int hd, int sl, at_f4 v) {
+    if constexpr (CAUSAL) {
+        const int K = a.H * D;
+        if constexpr (PAIR) {
+            wf_put2(a.planes, s, hd * D + (sl >> 1), K, v[0], v[2]);
+            wf_put2(a.planes, s, hd * D + (sl >> 1) + 64, K, v[1], v[3]);
+        } else {
+            wf_put4(a.planes, s, hd * D + sl, K, make_float4(v[0], v[1], v[2], v[3]));
+        }
+    } else {
+        *(at_f4*)(a.out + b * a.o_b + (int64_t)s * a.o_s + hd * D + sl) = v;
+    }
 }
 
 template <int D, typename KT, bool CAUSAL>
@@ -309,18 +326,12 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams 
         }
         const float inv = 1.0f / cl;
         const int s = (c0 + c) / p.G, hd = g * p.G + (c0 + c) - s * p.G;
-        float* orow = a.out + b * a.o_b + (int64_t)s * a.o_s + hd * D;
-        if constexpr (PAIR) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) orow[at_dim<PAIR>(sl + e)] = v[e] * inv;
-        } else {
-            *(at_f4*)(orow + sl) = v * inv;
-        }
+        at_store<PAIR, CAUSAL>(a, D, b, s, hd, sl, v * inv);
     }
 }
 
 // One column per D / 4 threads: the key splits' (max, sum, O) merged, in split order.
-template <int D, bool PAIR>
+template <int D, bool PAIR, bool CAUSAL>
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
     constexpr int TPC = D / 4;
     const AttnArgs& a = p.a;
@@ -344,13 +355,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
     }
     const float inv = 1.0f / l;
     const int s = c / p.G, hd = g * p.G + c - s * p.G;
-    float* orow = a.out + b * a.o_b + (int64_t)s * a.o_s + hd * D;
-    if constexpr (PAIR) {
-#pragma unroll
-        for (int e = 0; e < 4; e++) orow[at_dim<PAIR>(sl + e)] = v[e] * inv;
-    } else {
-        *(at_f4*)(orow + sl) = v * inv;
-    }
+    at_store<PAIR, CAUSAL>(a, D, b, s, hd, sl, v * inv);
 }
 
 bool attn_mfma_supported(const AttnArgs& a) {
@@ -372,7 +377,7 @@ static int attn_launch(AttnParams& p, hipStream_t st) {
     PIO_LAUNCHED();
     if (p.splits > 1) {
         const int64_t cols = (int64_t)a.B * a.Hk * a.S * p.G;
-        attn_merge_kernel<D, sizeof(KT) == 2><<<ceil_div(cols, 256 / (D / 4)), 256, 0, st>>>(p);
+        attn_merge_kernel<D, sizeof(KT) == 2, CAUSAL><<<ceil_div(cols, 256 / (D / 4)), 256, 0, st>>>(p);
         PIO_LAUNCHED();
     }
     return PIO_OK;

@@ -12,6 +12,7 @@ struct AttnArgs {
     const void* k;        // row (b, t) of kv head g: k + b * kv_b + t * kv_t + g * kv_h (elements)
     const void* v;        // as k
     float* out;           // row (b, s): out + b * o_b + s * o_s, head h at h * D (may be q itself)
+    int8_t* planes;       // causal: instead of out, the planes of row s (wf_planes.hpp, K = H * D)
     int64_t q_b, o_b, kv_b;
     int q_s, o_s, kv_t;
     int64_t kv_h;

@@ -847,8 +847,8 @@ static int launch_gemv_mfma(const _Float16* x, const int8_t* w, const float* s_w
 }
 
 // The W8 linear on the matrix cores (gemm_w8f.hip), for more than 4 rows.
-int gemm_w8f(const void* x, int x_dtype, int64_t ldx, const int8_t* w, const float* s_w, const float* bias,
-             void* y, int y_dtype, int64_t ldy, int M, int N, int K, bool resid, hipStream_t st);
+int gemm_w8f(const void* x, int x_dtype, const int8_t* w, const float* s_w, const float* bias, void* y, int y_dtype,
+             int M, int N, int K, hipStream_t st);
 constexpr int GEMV_MAX_FMA_ROWS = 4;
 
 // Below this weight size a launch is bounded by its start-up (one HBM round
@@ -868,8 +868,8 @@ static int dispatch(const XT* x, const int8_t* w, const float* s_w, const float*
     // More rows than one FMA launch serves: the MFMA GEMM reads W once, where
     // the FMA kernels would re-stream it every few rows.
     if (M > GEMV_MAX_FMA_ROWS)
-        return gemm_w8f(x, std::is_same<XT, float>::value ? PIO_F32 : PIO_F16, K, w, s_w, bias, y,
-                        std::is_same<YT, float>::value ? PIO_F32 : PIO_F16, N, M, N, K, false, st);
+        return gemm_w8f(x, std::is_same<XT, float>::value ? PIO_F32 : PIO_F16, w, s_w, bias, y,
+                        std::is_same<YT, float>::value ? PIO_F32 : PIO_F16, M, N, K, st);
     if ((size_t)N * K >= GEMV_STREAM_MIN_BYTES && stream_pick(1, N, K)) {
         // x rows in launches of up to 4 (as many as the LDS takes); each launch re-streams W
         for (int m0 = 0; m0 < M;) {

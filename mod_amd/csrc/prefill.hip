@@ -21,17 +21,15 @@
 // so decode steps and the persistent decode continue from it.
 #include "attention.hpp"
 #include "decode.hpp"
+#include "wf_planes.hpp"
 
 #include <float.h>
 #include <math.h>
 
 namespace pio {
 
-int gemm_w8f(const void* x, int x_dtype, int64_t ldx, const int8_t* w, const float* s_w, const float* bias,
-             void* y, int y_dtype, int64_t ldy, int M, int N, int K, bool resid, hipStream_t st);
-int gemm_w8f_split(const float* x, int64_t ldx, const int8_t* w, const float* s_w, const float* bias, float* y,
-                   int64_t ldy, int M, int N, int K, bool resid, Scratch& ws, const float** part, int* splits,
-                   hipStream_t st);
+int gemm_w8_planes(const int8_t* xp, const int8_t* w, const float* s_w, const float* bias, float* y, int64_t ldy, int M,
+                   int N, int K, bool resid, Scratch& ws, const float** part, int* splits, hipStream_t st);
 
 // x[m] = embed[ids[pos0 + m]] (an out-of-range id reads row 0, as the step).
 __global__ __launch_bounds__(256) void pf_embed_kernel(const float* __restrict__ embed, const int32_t* __restrict__ ids,
@@ -44,27 +42,35 @@ __global__ __launch_bounds__(256) void pf_embed_kernel(const float* __restrict__
     for (int i = threadIdx.x; i < H / 4; i += 256) dst[i] = src[i];
 }
 
-// h[m] = x[m] * (1 / sqrt(mean(x[m]^2) + eps)) * w, one block per row.
-__global__ __launch_bounds__(256) void pf_rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                         float* __restrict__ h, int H, float eps) {
+// The RMSNorm of row m, x[m] * (1 / sqrt(mean(x[m]^2) + eps)) * w, into the
+// planes of h, given the thread's sum of squares (256 threads; H % 4 == 0).
+__device__ __forceinline__ void pf_norm_row(const float* xr, const float* __restrict__ w, int8_t* __restrict__ h, int m,
+                                            int H, float eps, float ss) {
     __shared__ float red[4];
-    const int m = blockIdx.x, tid = threadIdx.x;
-    const float* xr = x + (int64_t)m * H;
-    float ss = 0.f;
-    for (int i = tid * 4; i < H; i += 1024) {
-        const float4 a = *(const float4*)(xr + i);
-        ss += a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w;
-    }
+    const int tid = threadIdx.x;
     ss = wave_sum(ss);
     if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
     const float r = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)H + eps);
-    float* hr = h + (int64_t)m * H;
     for (int i = tid * 4; i < H; i += 1024) {
         const float4 a = *(const float4*)(xr + i);
         const float4 g = *(const float4*)(w + i);
-        *(float4*)(hr + i) = make_float4(a.x * r * g.x, a.y * r * g.y, a.z * r * g.z, a.w * r * g.w);
+        wf_put4(h, m, i, H, make_float4(a.x * r * g.x, a.y * r * g.y, a.z * r * g.z, a.w * r * g.w));
     }
+}
+
+// One block per row (wf_row_of_block).
+__global__ __launch_bounds__(256) void pf_rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                         int8_t* __restrict__ h, int M, int H, float eps) {
+    const int m = wf_row_of_block(blockIdx.x);
+    if (m >= M) return;
+    const float* xr = x + (int64_t)m * H;
+    float ss = 0.f;
+    for (int i = threadIdx.x * 4; i < H; i += 1024) {
+        const float4 a = *(const float4*)(xr + i);
+        ss += a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w;
+    }
+    pf_norm_row(xr, w, h, m, H, eps, ss);
 }
 
 // Rotate-half RoPE at each row's position on the q and k heads of qkv (row m,
@@ -146,34 +152,45 @@ __global__ __launch_bounds__(64) void pf_qkv_finish_kernel(const float* __restri
     pf_rope_kv_put<KT>(qkv, ldq, pos0, nq, nkv, cos_t, sin_t, kc, vc, max_seq, m, head, i, a, b);
 }
 
-// The gate_up linear's K slices finished with SwiGLU: act[m][i] = silu(g) * u
-// for g, u formed as the GEMM's reduce forms them (no bias), the arithmetic of
-// pf_swiglu_kernel.
-__global__ __launch_bounds__(256) void pf_gu_finish_kernel(const float* __restrict__ part, int splits, int M, int I,
-                                                           const float* __restrict__ s_w, float* __restrict__ act) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (int64_t)M * I) return;
-    const int64_t m = e / I, i = e - m * I, MN = (int64_t)M * 2 * I, r = m * 2 * I;
-    float g = 0.f, u = 0.f;
-#pragma unroll 8
-    for (int z = 0; z < splits; z++) {
-        g += part[z * MN + r + i];
-        u += part[z * MN + r + I + i];
+// act[m][i] = silu(g) * u into the planes of act, 4 channels per thread, row m =
+// wf_row_of_block(blockIdx.y). part: g and u are the gate_up linear's K slices,
+// formed as the GEMM's reduce forms them (no bias); else the rows of gu.
+__device__ __forceinline__ float pf_silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
+__global__ __launch_bounds__(256) void pf_swiglu_kernel(const float* __restrict__ gu, const float* __restrict__ part,
+                                                        int splits, int M, int I, const float* __restrict__ s_w,
+                                                        int8_t* __restrict__ act) {
+    const int m = wf_row_of_block(blockIdx.y), i = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (m >= M || i >= I) return;
+    const int64_t r = (int64_t)m * 2 * I + i, MN = (int64_t)M * 2 * I;
+    float4 g, u;
+    if (part) {
+        const float4 sg = *(const float4*)(s_w + i), su = *(const float4*)(s_w + I + i);
+        g = u = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+        for (int z = 0; z < splits; z++) {
+            const float4 a = *(const float4*)(part + z * MN + r), c = *(const float4*)(part + z * MN + r + I);
+            g.x += a.x; g.y += a.y; g.z += a.z; g.w += a.w;
+            u.x += c.x; u.y += c.y; u.z += c.z; u.w += c.w;
+        }
+        g.x *= sg.x; g.y *= sg.y; g.z *= sg.z; g.w *= sg.w;
+        u.x *= su.x; u.y *= su.y; u.z *= su.z; u.w *= su.w;
+    } else {
+        g = *(const float4*)(gu + r);
+        u = *(const float4*)(gu + r + I);
     }
-    g = g * s_w[i];
-    u = u * s_w[I + i];
-    act[e] = g / (1.0f + expf(-g)) * u;
+    wf_put4(act, m, i, I, make_float4(pf_silu_mul(g.x, u.x), pf_silu_mul(g.y, u.y), pf_silu_mul(g.z, u.z),
+                                      pf_silu_mul(g.w, u.w)));
 }
 
 // A residual linear's K slices finished into x (x += slices * s, as the
 // GEMM's reduce forms it), then -- when w is given -- the RMSNorm of the new
-// row into h with pf_rmsnorm_kernel's arithmetic. One block per row; H % 4 == 0.
+// row into the planes of h. One block per row (wf_row_of_block); H % 4 == 0.
 __global__ __launch_bounds__(256) void pf_resid_norm_kernel(const float* __restrict__ part, int splits, int M, int H,
                                                             const float* __restrict__ s_w, float* __restrict__ x,
-                                                            const float* __restrict__ w, float* __restrict__ h,
+                                                            const float* __restrict__ w, int8_t* __restrict__ h,
                                                             float eps) {
-    __shared__ float red[4];
-    const int m = blockIdx.x, tid = threadIdx.x;
+    const int m = wf_row_of_block(blockIdx.x), tid = threadIdx.x;
+    if (m >= M) return;
     const int64_t MN = (int64_t)M * H;
     float* xr = x + (int64_t)m * H;
     float ss = 0.f;
@@ -196,29 +213,7 @@ __global__ __launch_bounds__(256) void pf_resid_norm_kernel(const float* __restr
         *(float4*)(xr + i) = a;
         ss += a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w;
     }
-    if (!w) return;
-    ss = wave_sum(ss);
-    if ((tid & 63) == 0) red[tid >> 6] = ss;
-    __syncthreads();
-    const float r = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)H + eps);
-    float* hr = h + (int64_t)m * H;
-    for (int i = tid * 4; i < H; i += 1024) {
-        const float4 a = *(const float4*)(xr + i);
-        const float4 g = *(const float4*)(w + i);
-        *(float4*)(hr + i) = make_float4(a.x * r * g.x, a.y * r * g.y, a.z * r * g.z, a.w * r * g.w);
-    }
-}
-
-constexpr int ATT_MAX_G_PF = 4;   // query heads per KV head
-
-// act[m][i] = silu(g) * u with g = gu[m][i], u = gu[m][I + i].
-__global__ __launch_bounds__(256) void pf_swiglu_kernel(const float* __restrict__ gu, float* __restrict__ act, int M,
-                                                        int I) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (int64_t)M * I) return;
-    const int64_t m = e / I, i = e - m * I;
-    const float g = gu[m * 2 * I + i], u = gu[m * 2 * I + I + i];
-    act[e] = g / (1.0f + expf(-g)) * u;
+    if (w) pf_norm_row(xr, w, h, m, H, eps, ss);
 }
 
 // The decoder's x = row `m` of the batch, and its position = pos (so that
@@ -228,6 +223,8 @@ __global__ void pf_handoff_kernel(const float* __restrict__ xb, int m, int H, fl
     for (int i = threadIdx.x; i < H; i += blockDim.x) x[i] = xb[(int64_t)m * H + i];
     if (threadIdx.x == 0) state[0] = pos;
 }
+
+constexpr int ATT_MAX_G_PF = 4;   // query heads per KV head
 
 int prefill(Qwen3Dec* d, int M, bool logits) {
     const pio_qwen3_config& c = d->c;
@@ -240,23 +237,28 @@ int prefill(Qwen3Dec* d, int M, bool logits) {
                 ATT_MAX_G_PF);
     PIO_REQUIRE(H % 16 == 0 && I % 16 == 0, "pio_qwen3_prefill: hidden and intermediate must be multiples of 16");
     hipStream_t st = d->st;
-    // activations of the batch: x, h (normed), qkv, attention out, [g|u], act
-    const size_t n_x = (size_t)M * H, n_qkv = (size_t)M * nqkv, n_o = (size_t)M * nq * D;
-    const size_t n_gu = (size_t)M * 2 * I, n_act = (size_t)M * I;
+    // activations of the batch: x, qkv and [g|u] in fp32; the linears' inputs (h,
+    // the normed x; the attention's output; act) as planes
+    auto al = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t b_x = al((size_t)M * H * 4), b_qkv = al((size_t)M * nqkv * 4), b_gu = al((size_t)M * 2 * I * 4);
+    const size_t b_h = al(wf_planes_bytes(M, H)), b_o = al(wf_planes_bytes(M, nq * D)), b_act = al(wf_planes_bytes(M, I));
     Scratch ws;
-    PIO_TRY(ws.get((2 * n_x + n_qkv + n_o + n_gu + n_act) * sizeof(float), st));
-    float* x = (float*)ws.ptr;
-    float* h = x + n_x;
-    float* qkv = h + n_x;
-    float* o = qkv + n_qkv;
-    float* gu = o + n_o;
-    float* act = gu + n_gu;
+    PIO_TRY(ws.get(b_x + b_qkv + b_gu + b_h + b_o + b_act, st));
+    char* at_ = (char*)ws.ptr;
+    auto take = [&](size_t b) { char* r = at_; at_ += b; return r; };
+    float* x = (float*)take(b_x);
+    float* qkv = (float*)take(b_qkv);
+    float* gu = (float*)take(b_gu);
+    int8_t* h = (int8_t*)take(b_h);
+    int8_t* o = (int8_t*)take(b_o);
+    int8_t* act = (int8_t*)take(b_act);
+    const int rb = wf_row_blocks(M);
     pf_embed_kernel<<<M, 256, 0, st>>>(d->embed, d->ids, pos0, x, H, c.vocab);
     PIO_LAUNCHED();
     // the causal attention of every layer: queries in the qkv rows, the cache's
     // rows [kv head][max_seq][D] for the layer
     AttnArgs at{};
-    at.q = qkv; at.out = o;
+    at.q = qkv; at.planes = o;
     at.q_s = nqkv; at.o_s = nq * D; at.kv_t = D; at.kv_h = (int64_t)c.max_seq * D;
     at.B = 1; at.S = M; at.T = pos0 + M; at.H = nq; at.Hk = nkv; at.D = D;
     at.scale = 1.0f / sqrtf((float)D);
@@ -273,14 +275,14 @@ int prefill(Qwen3Dec* d, int M, bool logits) {
         const pio_qwen3_layer& L = d->layers[l];
         const int64_t lkv = (int64_t)l * nkv * c.max_seq * D;   // elements
         if (!h_ready) {
-            pf_rmsnorm_kernel<<<M, 256, 0, st>>>(x, L.in_norm, h, H, c.rms_eps);
+            pf_rmsnorm_kernel<<<rb, 256, 0, st>>>(x, L.in_norm, h, M, H, c.rms_eps);
             PIO_LAUNCHED();
         }
         {
             Scratch pw;
             const float* part;
             int sp;
-            PIO_TRY(gemm_w8f_split(h, H, L.w_qkv, L.s_qkv, L.b_qkv, qkv, nqkv, M, nqkv, H, false, pw, &part, &sp, st));
+            PIO_TRY(gemm_w8_planes(h, L.w_qkv, L.s_qkv, L.b_qkv, qkv, nqkv, M, nqkv, H, false, pw, &part, &sp, st));
             const dim3 g(M, nq + 2 * nkv);
             if (d->kv16) {
                 _Float16* kc = (_Float16*)d->kc + lkv;
@@ -312,33 +314,30 @@ int prefill(Qwen3Dec* d, int M, bool logits) {
             Scratch pw;
             const float* part;
             int sp;
-            PIO_TRY(gemm_w8f_split(o, nq * D, L.w_o, L.s_o, nullptr, x, H, M, H, nq * D, true, pw, &part, &sp, st));
+            PIO_TRY(gemm_w8_planes(o, L.w_o, L.s_o, nullptr, x, H, M, H, nq * D, true, pw, &part, &sp, st));
             if (sp)
-                pf_resid_norm_kernel<<<M, 256, 0, st>>>(part, sp, M, H, L.s_o, x, L.post_norm, h, c.rms_eps);
+                pf_resid_norm_kernel<<<rb, 256, 0, st>>>(part, sp, M, H, L.s_o, x, L.post_norm, h, c.rms_eps);
             else
-                pf_rmsnorm_kernel<<<M, 256, 0, st>>>(x, L.post_norm, h, H, c.rms_eps);
+                pf_rmsnorm_kernel<<<rb, 256, 0, st>>>(x, L.post_norm, h, M, H, c.rms_eps);
             PIO_LAUNCHED();
         }
         {
             Scratch pw;
             const float* part;
             int sp;
-            PIO_TRY(gemm_w8f_split(h, H, L.w_gu, L.s_gu, nullptr, gu, 2 * I, M, 2 * I, H, false, pw, &part, &sp, st));
-            if (sp)
-                pf_gu_finish_kernel<<<ceil_div((int64_t)M * I, 256), 256, 0, st>>>(part, sp, M, I, L.s_gu, act);
-            else
-                pf_swiglu_kernel<<<ceil_div((int64_t)M * I, 256), 256, 0, st>>>(gu, act, M, I);
+            PIO_TRY(gemm_w8_planes(h, L.w_gu, L.s_gu, nullptr, gu, 2 * I, M, 2 * I, H, false, pw, &part, &sp, st));
+            pf_swiglu_kernel<<<dim3(ceil_div(I, 1024), rb), 256, 0, st>>>(gu, sp ? part : nullptr, sp, M, I, L.s_gu, act);
             PIO_LAUNCHED();
         }
         {
             Scratch pw;
             const float* part;
             int sp;
-            PIO_TRY(gemm_w8f_split(act, I, L.w_down, L.s_down, nullptr, x, H, M, H, I, true, pw, &part, &sp, st));
+            PIO_TRY(gemm_w8_planes(act, L.w_down, L.s_down, nullptr, x, H, M, H, I, true, pw, &part, &sp, st));
             const bool next = l + 1 < c.n_layers;
             h_ready = sp && next;
             if (sp) {
-                pf_resid_norm_kernel<<<M, 256, 0, st>>>(part, sp, M, H, L.s_down, x,
+                pf_resid_norm_kernel<<<rb, 256, 0, st>>>(part, sp, M, H, L.s_down, x,
                                                         next ? d->layers[l + 1].in_norm : nullptr, h, c.rms_eps);
                 PIO_LAUNCHED();
             }

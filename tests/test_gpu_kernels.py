@@ -818,3 +818,48 @@ def test_skinny_paths_full_size_properties(env):
     assert np.array_equal(host(accn), -ha)
     rows = [0, 1, 77, 4095, 100000, N - 1]
     assert np.array_equal(ha[:, rows], oracle.matmul_nt_i32(q, W[rows]))
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (9, 16400, 4112),     # 32 x 128 tiles; a last K step of 16
+    (33, 9001, 2064),     # 64 x 64 tiles, K slices
+    (129, 5003, 1040),    # 128 x 64: one row and 11 columns in the last tiles
+    (420, 6200, 1040),    # 128 x 128
+    (1000, 1000, 12304),  # two chunks of rows; one slice of K longer than the rest
+])
+def test_w8_linear_planes(env, M, N, K):
+    """fp32 x split into planes before the GEMM, at the edges of every tile shape
+    it picks. Random x against float64 within the bound of its roundings (one
+    per part and 16 products, 2^-23 each, on sums no larger than sum |x w|);
+    then one-hot weights and x with all 24 significand bits over 2^-20 .. 2^20,
+    where y is x itself, exactly."""
+    torch, ops, d = env
+    _say(f"W8 planes M={M} N={N} K={K}")
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=g)
+    W = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    s, b = torch.rand(N, generator=g) * 0.02 + 0.001, torch.randn(N, generator=g)
+    xd, Wd, sd, bd = (t.to(d) for t in (x, W, s, b))
+    y = torch.empty((M, N), device=d)
+    sync(torch)
+    ops.gemv_w8(xd, Wd, sd, bd, y, M, N, K)
+    sync(torch)
+    ref = (xd.double() @ Wd.double().t()) * sd.double() + bd.double()
+    mag = (xd.double().abs() @ Wd.double().abs().t()) * sd.double() + bd.double().abs()
+    bound = (3 * K / 16 + 8) * 2.0 ** -23 * mag
+    assert bool(((y.double() - ref).abs() <= bound).all())
+    x = torch.ldexp(torch.randint(2 ** 23, 2 ** 24, (M, K), generator=g).float(),
+                    torch.randint(-43, -3, (M, K), generator=g))
+    at = torch.arange(N) % K
+    sign = 1 - 2 * (torch.arange(N) % 2)
+    W = torch.zeros((N, K), dtype=torch.int8)
+    W[torch.arange(N), at] = sign.to(torch.int8)
+    xd, Wd, one = x.to(d), W.to(d), torch.full((N,), 4.0).to(d)
+    y16 = torch.empty((M, N), device=d, dtype=torch.float16)
+    sync(torch)
+    ops.gemv_w8(xd, Wd, one, None, y, M, N, K)
+    ops.gemv_w8(xd, Wd, one, None, y16, M, N, K)
+    sync(torch)
+    want = 4 * x[:, at] * sign
+    assert torch.equal(y.cpu(), want)
+    assert torch.equal(y16.cpu(), want.half())
