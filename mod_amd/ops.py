@@ -211,23 +211,33 @@ def check(status: int, what: str = "") -> None:
 
 def _ptr(x) -> int | None:
     """Device pointer of a torch tensor / int / None."""
-    if x is None:
-        return None
-    if isinstance(x, int):
+    if x is None or type(x) is int:
         return x
-    if hasattr(x, "data_ptr"):
-        return int(x.data_ptr())
-    raise TypeError(f"cannot take a device pointer of {type(x)}")
+    try:
+        return x.data_ptr()
+    except AttributeError:
+        if isinstance(x, int):
+            return x
+        raise TypeError(f"cannot take a device pointer of {type(x)}") from None
+
+
+# dtype object -> element-type code, filled as dtypes are seen: forming the
+# name for each argument was 1.3 us of a 5.3 us call whose kernel takes 2.9
+_dtype_seen: dict = {}
 
 
 def _dt(x, default=F32) -> int:
     """Element-type code of a torch tensor (or the default for raw pointers)."""
-    if hasattr(x, "dtype"):
-        name = str(x.dtype).replace("torch.", "")
-        if name in _DTYPE_CODES:
-            return _DTYPE_CODES[name]
-        raise TypeError(f"unsupported dtype {x.dtype}")
-    return default
+    d = getattr(x, "dtype", None)
+    if d is None:
+        return default
+    code = _dtype_seen.get(d)
+    if code is None:
+        name = str(d).replace("torch.", "")
+        if name not in _DTYPE_CODES:
+            raise TypeError(f"unsupported dtype {d}")
+        code = _dtype_seen[d] = _DTYPE_CODES[name]
+    return code
 
 
 def _stream(s) -> int | None:
