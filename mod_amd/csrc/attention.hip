@@ -23,13 +23,13 @@
 // of both in flight spilled registers: 88 us against 72 in the first case
 // below). The columns' q is in LDS. The waves' (max, sum, O) meet in LDS at
 // the end. When there are too few column tiles
-// for the CUs (decode steps: B * Hk tiles), the keys are split over workgroups
-// as well and a second launch merges the partials; such a launch is bound by
-// reading K and V, and the idle columns of its MFMAs cost no time.
+// for the CUs, the keys are split over workgroups as well and a second launch
+// merges the partials. Steps of at most AT_VEC_COLS columns per kv head run on
+// the VALU (attn_vec_kernel).
 //
 // Measured (MI355X; before: a workgroup per query row on the VALU, keys one by
 // one): 777 queries and keys, 16 heads over 8, D 128: 909 -> 72 us; one query
-// of 4 sequences over 2047 keys: 578 -> 27 us (2.5 TB/s); causal over 1021
+// of 4 sequences over 2047 keys: 578 -> 27 us (18 on the VALU kernel); causal over 1021
 // positions: 462 -> 57 us. Bound by the fp32 MFMA (35 us of it in the first)
 // and by the softmax between its two products, which two waves per SIMD only
 // partly cover. Error against 64 bits 3.1e-7 (was 5.2e-7) and 2.3e-7 (8.2e-7).
@@ -50,6 +50,7 @@ typedef _Float16 at_h8 __attribute__((ext_vector_type(8)));
 constexpr int AT_COLS = 32;    // (query, head) pairs per workgroup
 constexpr int AT_KEYS = 32;    // keys per tile
 constexpr int AT_WAVES = 4;
+constexpr int AT_VEC_COLS = 4; // columns per kv head up to which the VALU kernel serves
 
 struct AttnParams {
     AttnArgs a;
@@ -104,7 +105,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams 
     extern __shared__ __attribute__((aligned(16))) float at_lds[];
     __shared__ float at_m[AT_WAVES][AT_COLS], at_l[AT_WAVES][AT_COLS];
     const AttnArgs& a = p.a;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, h = lane >> 5;
 
     // kv heads fastest: with 8 of them each XCD's L2 holds one head's K and V
@@ -330,32 +331,207 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams 
     }
 }
 
-// One column per D / 4 threads: the key splits' (max, sum, O) merged, in split order.
+// Few columns (a decode step): the same split of keys over waves and
+// workgroups, on the VALU. A launch is bound by reading K and V, and the MFMAs
+// above would spend 32 columns' time on them: 4 sequences x 2047 keys, 2 heads
+// per kv head, 20.3 us (8 of them MFMAs) against 15.1 here (4.4 TB/s); 16 x 4000
+// keys run at 5.3 TB/s. Lane (i, h) holds
+// half h of key i's K row and slots NT i .. of half of the tile's V rows, loaded
+// as above; a score is summed over the two halves, the weights go through LDS
+// to the lanes of the V rows. K and V of the next tile are loaded as soon as this
+// one's registers are free.
+template <int D, int C>
+__global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_vec_kernel(AttnParams p) {
+    constexpr int NT = D / 32, KL = D / 8;
+    typedef typename AtRaw<float, D>::v at_vt;
+    __shared__ __attribute__((aligned(16))) float qs[C][D], ps[AT_WAVES][C][AT_KEYS], ob[AT_WAVES][C][D];
+    __shared__ float at_m[AT_WAVES][C], at_l[AT_WAVES][C];
+    const AttnArgs& a = p.a;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 31, h = lane >> 5;
+    const int g = blockIdx.x % a.Hk, b = blockIdx.x / a.Hk, ncols = a.S * p.G;
+    const int kt1 = min((int)(blockIdx.y + 1) * p.per_split, (a.T + AT_KEYS - 1) / AT_KEYS);
+    const float* kb = (const float*)a.k + b * a.kv_b + g * a.kv_h;
+    const float* vb = (const float*)a.v + b * a.kv_b + g * a.kv_h;
+    at_f4 kr[KL];
+    at_vt vr[16];
+    auto load_k = [&](int kt) {   // rows past the last key re-read it
+        const float* r = kb + (int64_t)min(kt * AT_KEYS + i, a.T - 1) * a.kv_t + 4 * h;
+#pragma unroll
+        for (int c = 0; c < KL; c++) kr[c] = *(const at_f4*)(r + 8 * c);
+    };
+    auto load_v = [&](int kt) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const int t = min(kt * AT_KEYS + 8 * (e >> 2) + 4 * h + (e & 3), a.T - 1);
+            vr[e] = *(const at_vt*)(vb + (int64_t)t * a.kv_t + NT * i);
+        }
+    };
+    int kt = blockIdx.y * p.per_split + w;
+    if (kt < kt1) {
+        load_k(kt);
+        load_v(kt);
+    }
+    for (int e = tid; e < C * (D / 4); e += 64 * AT_WAVES) {
+        const int c = min(e / (D / 4), ncols - 1), sl = (e % (D / 4)) * 4, s = c / p.G, hd = g * p.G + c - s * p.G;
+        *(at_f4*)&qs[e / (D / 4)][sl] = *(const at_f4*)(a.q + b * a.q_b + (int64_t)s * a.q_s + hd * D + sl);
+    }
+    __syncthreads();
+    float m[C], l[C], o[C][NT];
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        m[c] = a.m_seed;
+        l[c] = 0.f;
+#pragma unroll
+        for (int n = 0; n < NT; n++) o[c][n] = 0.f;
+    }
+    for (; kt < kt1; kt += AT_WAVES) {
+        const int t0 = kt * AT_KEYS;
+        const bool live = t0 + i < a.T;
+        // q stays in LDS: hoisted out of the loop it would fill the registers
+        int qh = h;
+        asm volatile("" : "+v"(qh));
+        float s[C];
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            at_f4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < KL; k++) {
+                const at_f4 qv = ((const at_f4*)&qs[c][8 * k])[qh];
+#pragma unroll
+                for (int e = 0; e < 4; e++) d[e] = fmaf(kr[k][e], qv[e], d[e]);
+                if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // not all of q's reads at once
+            }
+            s[c] = (d[0] + d[1]) + (d[2] + d[3]);
+            asm volatile("" : "+v"(s[c]));   // formed here: sunk past the next loads, K would be held twice
+        }
+        if (kt + AT_WAVES < kt1) load_k(kt + AT_WAVES);
+        if (t0 + AT_KEYS > a.T) {
+            // a key past the last one: zero weight, and nothing inf or NaN in its row
+#pragma unroll
+            for (int e = 0; e < 16; e++)
+                if (t0 + 8 * (e >> 2) + 4 * h + (e & 3) >= a.T)
+#pragma unroll
+                    for (int n = 0; n < NT; n++) vr[e][n] = 0.f;
+        }
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            const float v = (s[c] + __shfl_xor(s[c], 32, 64)) * a.scale;
+            float mt = live ? v : a.m_seed;
+            mt = fmaxf(mt, dpp<DPP_XOR1>(mt));
+            mt = fmaxf(mt, dpp<DPP_XOR2>(mt));
+            mt = fmaxf(mt, dpp<DPP_HMIRROR>(mt));
+            mt = fmaxf(mt, dpp<DPP_MIRROR>(mt));
+            mt = fmaxf(m[c], fmaxf(rlane(mt, 0), rlane(mt, 16)));
+            const float pr = live ? expf(v - mt) : 0.f, corr = expf(m[c] - mt);
+            l[c] = l[c] * corr + pr;
+#pragma unroll
+            for (int n = 0; n < NT; n++) o[c][n] *= corr;
+            m[c] = mt;
+            if (h == 0) ps[w][c][i] = pr;
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int c = 0; c < C; c++)
+#pragma unroll
+            for (int e = 0; e < 16; e += 4) {
+                const at_f4 pr = *(const at_f4*)&ps[w][c][2 * e + 4 * h];
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+#pragma unroll
+                    for (int n = 0; n < NT; n++) o[c][n] = fmaf(pr[r], vr[e + r][n], o[c][n]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+        for (int c = 0; c < C; c++)
+#pragma unroll
+            for (int n = 0; n < NT; n++) asm volatile("" : "+v"(o[c][n]));   // as above, for V
+        if (kt + AT_WAVES < kt1) load_v(kt + AT_WAVES);
+    }
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const float ls = wsum(l[c]) * 0.5f;   // every key's weight is in both halves
+        if (lane == 0) {
+            at_m[w][c] = m[c];
+            at_l[w][c] = ls;
+        }
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+            const float t = o[c][n] + __shfl_xor(o[c][n], 32, 64);
+            if (h == 0) ob[w][c][NT * i + n] = t;
+        }
+    }
+    __syncthreads();
+    for (int e = tid; e < C * (D / 4); e += 64 * AT_WAVES) {
+        const int c = e / (D / 4), sl = (e % (D / 4)) * 4;
+        if (c >= ncols) continue;
+        float cm = at_m[0][c], cl = 0.f;
+#pragma unroll
+        for (int k = 1; k < AT_WAVES; k++) cm = fmaxf(cm, at_m[k][c]);
+        at_f4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < AT_WAVES; k++) {
+            const float f = expf(at_m[k][c] - cm);
+            cl += at_l[k][c] * f;
+            v += *(const at_f4*)&ob[k][c][sl] * f;
+        }
+        const int s = c / p.G;
+        if (p.splits > 1) {
+            const int64_t at = ((int64_t)blockIdx.y * a.B * a.Hk + blockIdx.x) * p.tiles * AT_COLS + c;
+            *(at_f4*)(p.part_o + at * D + sl) = v;
+            if (sl == 0) {
+                p.part_ml[2 * at] = cm;
+                p.part_ml[2 * at + 1] = cl;
+            }
+        } else {
+            at_store<false, false>(a, D, b, s, g * p.G + c - s * p.G, sl, v * (1.0f / cl));
+        }
+    }
+}
+
+// One column per block: the key splits' (max, sum, O) merged. Thread group z of
+// 256 / (D / 4) takes every such split, all loads of one in flight together (one
+// thread per 4 slots walking the splits in turn took 8 us for 16 of them).
 template <int D, bool PAIR, bool CAUSAL>
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
-    constexpr int TPC = D / 4;
+    constexpr int TPC = D / 4, Z = 256 / TPC;
+    __shared__ __attribute__((aligned(16))) float so[Z][D];
+    __shared__ float sm[Z], sl_[Z];
     const AttnArgs& a = p.a;
     const int ncols = a.S * p.G;
-    const int64_t i = (int64_t)blockIdx.x * (256 / TPC) + threadIdx.x / TPC;   // (b, kv head, column)
-    if (i >= (int64_t)a.B * a.Hk * ncols) return;
-    const int sl = (threadIdx.x % TPC) * 4;
-    const int64_t bg = i / ncols;
-    const int c = (int)(i - bg * ncols), b = (int)(bg / a.Hk), g = (int)(bg - (int64_t)b * a.Hk);
-    const int64_t step = (int64_t)a.B * a.Hk * p.tiles * AT_COLS, at = bg * p.tiles * AT_COLS + c;
-    float mx = p.part_ml[2 * at];
-#pragma unroll 8
-    for (int z = 1; z < p.splits; z++) mx = fmaxf(mx, p.part_ml[2 * (at + z * step)]);
-    float l = 0.f;
+    const int bg = blockIdx.x / ncols, c = blockIdx.x - bg * ncols, b = bg / a.Hk, g = bg - b * a.Hk;
+    const int zg = threadIdx.x / TPC, sl = (threadIdx.x % TPC) * 4;
+    const int64_t step = (int64_t)a.B * a.Hk * p.tiles * AT_COLS, at = (int64_t)bg * p.tiles * AT_COLS + c;
+    float m = -FLT_MAX, l = 0.f;
     at_f4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int z = 0; z < p.splits; z++) {
-        const float f = expf(p.part_ml[2 * (at + z * step)] - mx);
-        l += p.part_ml[2 * (at + z * step) + 1] * f;
-        v += *(const at_f4*)(p.part_o + (at + z * step) * D + sl) * f;
+#pragma unroll 2
+    for (int z = zg; z < p.splits; z += Z) {
+        const float zm = p.part_ml[2 * (at + z * step)], zl = p.part_ml[2 * (at + z * step) + 1];
+        const at_f4 zo = *(const at_f4*)(p.part_o + (at + z * step) * D + sl);
+        const float nm = fmaxf(m, zm), f = expf(m - nm), fz = expf(zm - nm);
+        l = l * f + zl * fz;
+        v = v * f + zo * fz;
+        m = nm;
     }
-    const float inv = 1.0f / l;
-    const int s = c / p.G, hd = g * p.G + c - s * p.G;
-    at_store<PAIR, CAUSAL>(a, D, b, s, hd, sl, v * inv);
+    *(at_f4*)&so[zg][sl] = v;
+    if (sl == 0) {
+        sm[zg] = m;
+        sl_[zg] = l;
+    }
+    __syncthreads();
+    if (zg) return;
+    const int nz = min(Z, p.splits);
+    float mx = sm[0];
+    for (int z = 1; z < nz; z++) mx = fmaxf(mx, sm[z]);
+    l = 0.f;
+    v = at_f4{0.f, 0.f, 0.f, 0.f};
+    for (int z = 0; z < nz; z++) {
+        const float f = expf(sm[z] - mx);
+        l += sl_[z] * f;
+        v += *(const at_f4*)&so[z][sl] * f;
+    }
+    const int s = c / p.G;
+    at_store<PAIR, CAUSAL>(a, D, b, s, g * p.G + c - s * p.G, sl, v * (1.0f / l));
 }
 
 bool attn_mfma_supported(const AttnArgs& a) {
@@ -367,20 +543,36 @@ bool attn_mfma_supported(const AttnArgs& a) {
     return aligned16(a.q) && aligned16(a.k) && aligned16(a.v) && aligned16(a.out);
 }
 
+template <int D, bool PAIR, bool CAUSAL>
+static int attn_merge(const AttnParams& p, hipStream_t st) {
+    if (p.splits == 1) return PIO_OK;
+    const AttnArgs& a = p.a;
+    attn_merge_kernel<D, PAIR, CAUSAL><<<(unsigned)((int64_t)a.B * a.Hk * a.S * p.G), 256, 0, st>>>(p);
+    PIO_LAUNCHED();
+    return PIO_OK;
+}
+
 template <int D, typename KT, bool CAUSAL>
-static int attn_launch(AttnParams& p, hipStream_t st) {
+static int attn_launch(const AttnParams& p, hipStream_t st) {
     const AttnArgs& a = p.a;
     const size_t lds = at_lds_bytes<D>();
     const dim3 grid((unsigned)((int64_t)p.tiles * a.B * a.Hk), p.splits);
     PIO_TRY((allow_lds<attn_mfma_kernel<D, KT, CAUSAL>>(lds)));
     attn_mfma_kernel<D, KT, CAUSAL><<<grid, 64 * AT_WAVES, lds, st>>>(p);
     PIO_LAUNCHED();
-    if (p.splits > 1) {
-        const int64_t cols = (int64_t)a.B * a.Hk * a.S * p.G;
-        attn_merge_kernel<D, sizeof(KT) == 2, CAUSAL><<<ceil_div(cols, 256 / (D / 4)), 256, 0, st>>>(p);
-        PIO_LAUNCHED();
-    }
-    return PIO_OK;
+    return attn_merge<D, sizeof(KT) == 2, CAUSAL>(p, st);
+}
+
+template <int D>
+static int attn_vec_launch(const AttnParams& p, hipStream_t st) {
+    const AttnArgs& a = p.a;
+    const dim3 grid(a.B * a.Hk, p.splits);
+    const int cols = a.S * p.G;
+    if (cols == 1) attn_vec_kernel<D, 1><<<grid, 64 * AT_WAVES, 0, st>>>(p);
+    else if (cols == 2) attn_vec_kernel<D, 2><<<grid, 64 * AT_WAVES, 0, st>>>(p);
+    else attn_vec_kernel<D, AT_VEC_COLS><<<grid, 64 * AT_WAVES, 0, st>>>(p);
+    PIO_LAUNCHED();
+    return attn_merge<D, false, false>(p, st);
 }
 
 int attn_mfma(const AttnArgs& a, hipStream_t st) {
@@ -404,6 +596,8 @@ int attn_mfma(const AttnArgs& a, hipStream_t st) {
         p.part_ml = p.part_o + cols * a.D;
     }
     if (a.causal) return a.kv16 ? attn_launch<128, _Float16, true>(p, st) : attn_launch<128, float, true>(p, st);
+    // measured at T = 1000, 8 kv heads: 8 columns 17.7 us here and 14.3 on the MFMAs
+    if (ncols <= AT_VEC_COLS) return a.D == 128 ? attn_vec_launch<128>(p, st) : attn_vec_launch<64>(p, st);
     return a.D == 128 ? attn_launch<128, float, false>(p, st) : attn_launch<64, float, false>(p, st);
 }
 

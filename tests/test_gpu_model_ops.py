@@ -125,7 +125,8 @@ def test_scaled_dot_product_attention(B, Bn, S, H, Hk, T, D):
     (1, 17, 2, 2, 128, 64),      # a tile of 32 with 17 columns; one key tile per wave
     (1, 11, 3, 1, 31, 128),      # 33 columns: the second tile holds one; a partial key tile
     (1, 65, 4, 4, 65, 64), (3, 1, 16, 8, 1023, 128),   # keys split over workgroups, ragged last split
-    (1, 300, 8, 2, 517, 128), (2, 1, 32, 4, 4100, 64)])
+    (1, 300, 8, 2, 517, 128), (2, 1, 32, 4, 4100, 64),
+    (2, 1, 8, 8, 70, 128), (1, 3, 2, 2, 33, 64), (1, 2, 4, 2, 2049, 128)])   # 1, 3 and 4 columns: the VALU kernel
 def test_attention_tiles(B, Bn, S, H, Hk, T, D):
     """The matrix-core attention at the edges of its column and key tiles and of
     its key splits, against the oracle and against the general kernel (which
