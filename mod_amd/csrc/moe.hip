@@ -24,6 +24,8 @@
 //  6. combine: out[t] = sum_{k=0..top_k-1} w[t,k] * down[pos(t,k)], in k order.
 #include "gemm_core.hpp"
 
+#include <algorithm>
+
 namespace pio {
 
 // Minimum over the 64 lanes (in every lane), on DPP lane moves and readlane.
@@ -113,35 +115,13 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
                 topk_id + (int64_t)t * top_k);
 }
 
-// The layer's first launch: block b takes tokens 2b and 2b + 1; waves 0-1
-// route them, waves 2-3 quantize their x rows per token (the quantizer of
-// quant.hip: amax / 127, IEEE division, round-half-even), each row loaded once
-// into registers, lane l holding the 8-element chunks l, l + 64, ...
-// (H % 8 == 0, H <= 512 ROUTE_XG).
+// Quantizer of one row by one wave (quant.hip's: amax / 127, IEEE division,
+// round-half-even), the row loaded once into registers, lane l holding the
+// 8-element chunks l, l + 64, ... (H % 8 == 0, H <= 512 ROUTE_XG).
 constexpr int ROUTE_XG = 8;
 template <typename XT>
-__global__ __launch_bounds__(256) void moe_route_quant_kernel(const float* __restrict__ logits,
-                                                              const XT* __restrict__ x, int H,
-                                                              float* __restrict__ topk_w,
-                                                              int32_t* __restrict__ topk_id,
-                                                              int8_t* __restrict__ qx,
-                                                              float* __restrict__ sx, int T,
-                                                              int E, int top_k, int renorm,
-                                                              unsigned* __restrict__ hmax) {
-    __shared__ float sp[2][ROUTE_MAX_E];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    // the gate_up epilogue's per-row max starts from 0 (grid >= 128 T threads >= T * top_k)
-    {
-        const int i = blockIdx.x * 256 + threadIdx.x;
-        if (i < T * top_k) hmax[i] = 0u;
-    }
-    const int t = blockIdx.x * 2 + (w & 1);
-    if (t >= T) return;
-    if (w < 2) {
-        route_token(logits + (int64_t)t * E, sp[w], lane, E, top_k, renorm,
-                    topk_w + (int64_t)t * top_k, topk_id + (int64_t)t * top_k);
-        return;
-    }
+__device__ __forceinline__ void quant_token(const XT* __restrict__ x, int t, int lane, int H, int8_t* __restrict__ qx,
+                                            float* __restrict__ sx) {
     const XT* xr = x + (int64_t)t * H;
     const int nch = H / 8;
     // every group's raw bits first (clamped chunk index), widened afterwards
@@ -171,6 +151,34 @@ __global__ __launch_bounds__(256) void moe_route_quant_kernel(const float* __res
             for (int i = 0; i < 4; i++) hi |= (uint32_t)(uint8_t)quant1(v[g][4 + i], sc) << (8 * i);
             *(uint2*)(qr + 8 * (lane + 64 * g)) = make_uint2(lo, hi);
         }
+}
+
+// The layer's first launch: block b takes tokens 2b and 2b + 1; waves 0-1
+// route them, waves 2-3 quantize their x rows per token.
+template <typename XT>
+__global__ __launch_bounds__(256) void moe_route_quant_kernel(const float* __restrict__ logits,
+                                                              const XT* __restrict__ x, int H,
+                                                              float* __restrict__ topk_w,
+                                                              int32_t* __restrict__ topk_id,
+                                                              int8_t* __restrict__ qx,
+                                                              float* __restrict__ sx, int T,
+                                                              int E, int top_k, int renorm,
+                                                              unsigned* __restrict__ hmax) {
+    __shared__ float sp[2][ROUTE_MAX_E];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    // the gate_up epilogue's per-row max starts from 0 (grid >= 128 T threads >= T * top_k)
+    {
+        const int i = blockIdx.x * 256 + threadIdx.x;
+        if (i < T * top_k) hmax[i] = 0u;
+    }
+    const int t = blockIdx.x * 2 + (w & 1);
+    if (t >= T) return;
+    if (w < 2) {
+        route_token(logits + (int64_t)t * E, sp[w], lane, E, top_k, renorm,
+                    topk_w + (int64_t)t * top_k, topk_id + (int64_t)t * top_k);
+        return;
+    }
+    quant_token<XT>(x, t, lane, H, qx, sx);
 }
 
 // ------------------------------------------------------------------ group ---
@@ -391,6 +399,224 @@ static void launch_grouped(const GroupedParams& g, dim3 grid, int nk, hipStream_
     }
 }
 
+// -------------------------------------------------------- one or two tokens ---
+// A decode step: the six launches above move the 8 experts' 38 MB in 14 us and
+// take 36, most of it launches, and blocks for every expert without a token.
+// Here one block routes, quantizes and groups the tokens (and lists the experts
+// that have any), and two weight-streaming kernels take the tokens of one expert:
+// a wave owns 16 weight rows (gate_up: 16 gate and the matching 16 up rows) and
+// loads them straight into registers in the operand layout of
+// v_mfma_i32_16x16x64_i8, two sets of MS_SET K values in flight, with the
+// activation rows in LDS; the down kernel quantizes its h rows itself. Same
+// integer sums, scales and order as above, so the same bits.
+// Qwen3-30B-A3B layer: T = 1 36.4 -> 25.2 us. From T = 3 the path above is the
+// faster one (41 / 46 us at 3, 86 / 114 at 16): these loads cover half a line of
+// a row each and stream at 4 TB/s, its tiles at 4.6 and up, and one block takes
+// longer to route many tokens than the launch it saves.
+constexpr int MS_MAX_T = 2;        // tokens (and rows of an expert)
+constexpr int MS_MAX_P = 64 * MS_MAX_T;   // (token, slot) pairs
+constexpr int MS_SET = 512;        // K values of a wave's rows per register set
+constexpr int MS_LOADS = MS_SET / 64;
+
+struct MoeFront {
+    const float* logits;
+    const void* x;
+    int H, T, E, top_k, renorm;
+    float* topk_w;
+    int32_t* topk_id;
+    int8_t* qx;
+    float* sx;
+    unsigned* hmax;
+    int32_t *offsets, *row_token, *pos_of_pair;
+    int32_t* active;               // [0] experts with tokens, then their ids
+};
+
+template <typename XT>
+__global__ __launch_bounds__(1024) void moe_front_kernel(MoeFront p) {
+    extern __shared__ float fr_p[];               // [T][E] probabilities
+    __shared__ __attribute__((aligned(16))) int32_t ids[MS_MAX_P];
+    __shared__ int32_t off[ROUTE_MAX_E];
+    __shared__ int wsum_[16];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, P = p.T * p.top_k;
+    for (int i = tid; i < P; i += 1024) p.hmax[i] = 0u;
+    // jobs 0 .. T-1 route a token, T .. 2T-1 quantize one
+    for (int j = w; j < 2 * p.T; j += 16) {
+        if (j < p.T) {
+            route_token(p.logits + (int64_t)j * p.E, fr_p + j * p.E, lane, p.E, p.top_k, p.renorm,
+                        p.topk_w + j * p.top_k, p.topk_id + j * p.top_k);
+        } else {
+            quant_token<XT>((const XT*)p.x, j - p.T, lane, p.H, p.qx, p.sx);
+        }
+    }
+    __syncthreads();   // and this block's topk_id writes are visible to it
+    const int P4 = (P + 3) & ~3;
+    if (tid < P4) ids[tid] = tid < P ? p.topk_id[tid] : 0x7fffffff;
+    __syncthreads();
+    // thread e: the pairs routed below expert e, and whether it has any
+    int below = 0, mine = 0;
+#pragma unroll 4
+    for (int i = 0; i < P4; i += 4) {
+        const v4i d = *(const v4i*)&ids[i];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            below += d[u] < tid;
+            mine |= d[u] == tid;
+        }
+    }
+    if (tid < p.E) {
+        p.offsets[tid] = below;
+        off[tid] = below;
+    }
+    if (tid == 0) p.offsets[p.E] = P;
+    const unsigned long long m = __ballot(mine > 0);
+    if (lane == 0) wsum_[w] = __popcll(m);
+    __syncthreads();
+    int rank = __popcll(m & ((1ull << lane) - 1ull)), all = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        rank += i < w ? wsum_[i] : 0;
+        all += wsum_[i];
+    }
+    if (mine) p.active[1 + rank] = tid;
+    if (tid == 0) p.active[0] = all;
+    // thread i: the row of pair i (pairs are in token order, so are an expert's rows)
+    if (tid < P) {
+        const int id = ids[tid];
+        int pos = off[id];
+#pragma unroll 4
+        for (int i = 0; i < P4; i += 4) {
+            const v4i d = *(const v4i*)&ids[i];
+#pragma unroll
+            for (int u = 0; u < 4; u++) pos += d[u] == id && i + u < tid;
+        }
+        p.row_token[pos] = tid / p.top_k;
+        p.pos_of_pair[tid] = pos;
+    }
+}
+
+typedef __attribute__((address_space(1))) const v4i ms_gv4i;
+
+struct MoeSmall {
+    const int32_t* active;
+    const int32_t* offsets;
+    const int32_t* row_token;
+    const int8_t* qx;         // gate_up: [T][K]
+    const float* sx;
+    const float* hin;         // down: h [pairs][K]
+    unsigned* amax;           // per pair: max |h| bits (gate_up writes, down reads)
+    const int8_t* W;          // [E][N][K]
+    const float* s_w;
+    float* out;               // gate_up: h [pairs][N / 2]; down: d [pairs][N]
+    int N, K;
+};
+
+// One wave per block (WGs of 4 waves: 29.9 us at T = 1); grid (N' / 16, min(E,
+// pairs)), N' = N / 2 channels or N rows, a multiple of 16.
+template <bool GU, int NS>
+__global__ __launch_bounds__(64) void moe_small_kernel(MoeSmall p) {
+    constexpr int R = GU ? 2 : 1;                       // 16-row weight blocks per wave
+    extern __shared__ __attribute__((aligned(16))) int8_t ms_lds[];
+    __shared__ float sa[MS_MAX_T];
+    if ((int)blockIdx.y >= p.active[0]) return;
+    const int e = p.active[1 + blockIdx.y];
+    const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
+    const int K = p.K, pitch = K + 16, NC = GU ? p.N / 2 : p.N;
+    const int n0 = blockIdx.x * 16, nr = n0 + r;
+    const int8_t* wp[R];
+    float sw[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const int64_t row = (int64_t)e * p.N + nr + j * NC;
+        wp[j] = p.W + row * K + 16 * q;
+        sw[j] = p.s_w[row];
+    }
+    v4i wr[NS < 2 ? 1 : 2][R][MS_LOADS];
+    auto load = [&](int s) {     // chunks past K re-read the last one (their products are skipped)
+#pragma unroll
+        for (int i = 0; i < MS_LOADS; i++)
+#pragma unroll
+            for (int j = 0; j < R; j++) wr[s & 1][j][i] = *(ms_gv4i*)(wp[j] + min(s * MS_SET + 64 * i, K - 64));
+    };
+    load(0);
+    if (NS > 1) load(1);
+    __builtin_amdgcn_sched_barrier(0);
+    const int beg = p.offsets[e], cnt = min(p.offsets[e + 1] - beg, MS_MAX_T);   // a token has an expert once
+    if (GU) {
+        // activation rows through the token list
+        for (int i = 0; i < cnt; i++) {
+            const int t = p.row_token[beg + i];
+            for (int c = lane; c < K / 16; c += 64)
+                *(v4i*)(ms_lds + i * pitch + 16 * c) = *(ms_gv4i*)(p.qx + (int64_t)t * K + 16 * c);
+            if (lane == 0) sa[i] = p.sx[t];
+        }
+    } else {
+        // h rows quantized with the row's max (the per-token quantizer's rule)
+        for (int i = 0; i < cnt; i++) {
+            const float am = __uint_as_float(p.amax[beg + i]), sc = am == 0.f ? 1.f : am / 127.0f;
+            const float4* h4 = (const float4*)(p.hin + (int64_t)(beg + i) * K);
+            for (int c = lane; c < K / 4; c += 64) {
+                const float4 v = h4[c];
+                *(uint32_t*)(ms_lds + i * pitch + 4 * c) =
+                    (uint32_t)(uint8_t)quant1(v.x, sc) | (uint32_t)(uint8_t)quant1(v.y, sc) << 8 |
+                    (uint32_t)(uint8_t)quant1(v.z, sc) << 16 | (uint32_t)(uint8_t)quant1(v.w, sc) << 24;
+            }
+            if (lane == 0) sa[i] = sc;
+        }
+    }
+    stage_barrier<63>();         // LDS written; the weight loads stay in flight
+    typedef int v4i_acc __attribute__((ext_vector_type(4)));
+    v4i_acc acc[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) acc[j] = v4i_acc{0, 0, 0, 0};
+    // rows past cnt read row 0 of the tile: their sums are dropped
+    const int8_t* as = ms_lds + (r < cnt ? r : 0) * pitch + 16 * q;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+#pragma unroll
+        for (int i = 0; i < MS_LOADS; i++) {
+            const int k = s * MS_SET + 64 * i;
+            if (s < NS - 1 || k < K) {
+                const v4i a = *(const v4i*)(as + k);
+#pragma unroll
+                for (int j = 0; j < R; j++)
+                    acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, wr[s & 1][j][i], acc[j], 0, 0, 0);
+            }
+        }
+        if (s + 2 < NS) load(s + 2);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // accumulator: activation rows 4 q + v, weight row r
+#pragma unroll
+    for (int v = 0; v < min(4, MS_MAX_T); v++) {
+        const int row = 4 * q + v;
+        if constexpr (GU) {
+            float h = 0.f;
+            if (row < cnt) h = silu_mul((float)acc[0][v] * sa[row] * sw[0], (float)acc[R - 1][v] * sa[row] * sw[R - 1]);
+            float mx = fabsf(h);   // over the 16 channels: 16 consecutive lanes
+            mx = fmaxf(mx, dpp<DPP_XOR1>(mx));
+            mx = fmaxf(mx, dpp<DPP_XOR2>(mx));
+            mx = fmaxf(mx, dpp<DPP_HMIRROR>(mx));
+            mx = fmaxf(mx, dpp<DPP_MIRROR>(mx));
+            if (row < cnt) {
+                p.out[(int64_t)(beg + row) * NC + n0 + r] = h;
+                if (r == 0) atomicMax(p.amax + beg + row, __float_as_uint(mx));
+            }
+        } else if (row < cnt) {
+            p.out[(int64_t)(beg + row) * NC + n0 + r] = (float)acc[0][v] * sa[row] * sw[0];
+        }
+    }
+}
+
+template <bool GU, int NS>
+static int launch_small(const MoeSmall& p, dim3 grid, int ns, hipStream_t st) {
+    if constexpr (NS * MS_SET <= 4096) {
+        if (ns != NS) return launch_small<GU, NS + 1>(p, grid, ns, st);
+        moe_small_kernel<GU, NS><<<grid, 64, (size_t)MS_MAX_T * (p.K + 16), st>>>(p);
+        PIO_LAUNCHED();
+    }
+    return PIO_OK;
+}
+
 // --------------------------------------------------------------- requant ---
 // Requantization of h per row: s = max|h| / 127 (1 when 0), q = rint(h / s)
 // clamped to +-127, the per-token quantizer's rule; max|h| comes from the
@@ -471,6 +697,7 @@ struct MoeWs {
     int32_t* offsets;
     int32_t* row_token;
     int32_t* pos_of_pair;
+    int32_t* active;     // [1 + MS_MAX_P], the path of one or two tokens
     int8_t* qx;
     float* sx;
     float* h;            // [P][I] SwiGLU output (fp32)
@@ -493,6 +720,7 @@ static MoeWs moe_layout(char* base, int T, int H, int I, int E, int k) {
     w.offsets = (int32_t*)take((size_t)(E + 1) * 4);
     w.row_token = (int32_t*)take(P * 4);
     w.pos_of_pair = (int32_t*)take(P * 4);
+    w.active = (int32_t*)take((size_t)(MS_MAX_P + 1) * 4);
     w.qx = (int8_t*)take((size_t)T * H);
     w.sx = (float*)take((size_t)T * 4);
     w.h = (float*)take(P * I * 4);
@@ -543,6 +771,30 @@ int moe_w8a8(const void* x, int x_dtype, const float* logits, const int8_t* w_gu
     MoeWs w = moe_layout((char*)ws, T, H, I, E, top_k);
     const int P = T * top_k;
 
+    auto combine = [&]() -> int {
+        dim3 cg(ceil_div(H, 1024), T);
+        if (out_dtype == PIO_F32)
+            moe_combine_kernel<float><<<cg, 256, 0, st>>>(w.d, w.topk_w, w.pos_of_pair, (float*)out, T, H, top_k);
+        else
+            moe_combine_kernel<_Float16><<<cg, 256, 0, st>>>(w.d, w.topk_w, w.pos_of_pair, (_Float16*)out, T, H, top_k);
+        PIO_LAUNCHED();
+        return PIO_OK;
+    };
+    if (T <= MS_MAX_T) {
+        MoeFront f{logits, x, H, T, E, top_k, renorm, w.topk_w, w.topk_id, w.qx, w.sx, w.amax, w.offsets, w.row_token,
+                   w.pos_of_pair, w.active};
+        const size_t lds = (size_t)T * E * sizeof(float);
+        if (x_dtype == PIO_F32) moe_front_kernel<float><<<1, 1024, lds, st>>>(f);
+        else moe_front_kernel<_Float16><<<1, 1024, lds, st>>>(f);
+        PIO_LAUNCHED();
+        const int na = std::min(E, P);
+        MoeSmall g{w.active, w.offsets, w.row_token, w.qx, w.sx, nullptr, w.amax, w_gu, s_gu, w.h, 2 * I, H};
+        PIO_TRY((launch_small<true, 1>(g, dim3(I / 16, na), ceil_div(H, MS_SET), st)));
+        MoeSmall d{w.active, w.offsets, w.row_token, nullptr, nullptr, w.h, w.amax, w_down, s_down, w.d, H, I};
+        PIO_TRY((launch_small<false, 1>(d, dim3(H / 16, na), ceil_div(I, MS_SET), st)));
+        return combine();
+    }
+
     if (x_dtype == PIO_F32)
         moe_route_quant_kernel<float><<<ceil_div(T, 2), 256, 0, st>>>(
             logits, (const float*)x, H, w.topk_w, w.topk_id, w.qx, w.sx, T, E, top_k, renorm, w.amax);
@@ -571,13 +823,7 @@ int moe_w8a8(const void* x, int x_dtype, const float* logits, const int8_t* w_gu
     launch_grouped<1, false>(d, dim3(ceil_div(H, MoeTile::BN), E), I / 128, st);
     PIO_LAUNCHED();
 
-    dim3 cg(ceil_div(H, 1024), T);
-    if (out_dtype == PIO_F32)
-        moe_combine_kernel<float><<<cg, 256, 0, st>>>(w.d, w.topk_w, w.pos_of_pair, (float*)out, T, H, top_k);
-    else
-        moe_combine_kernel<_Float16><<<cg, 256, 0, st>>>(w.d, w.topk_w, w.pos_of_pair, (_Float16*)out, T, H, top_k);
-    PIO_LAUNCHED();
-    return PIO_OK;
+    return combine();
 }
 
 }  // namespace pio

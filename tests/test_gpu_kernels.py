@@ -863,3 +863,36 @@ def test_w8_linear_planes(env, M, N, K):
     want = 4 * x[:, at] * sign
     assert torch.equal(y.cpu(), want)
     assert torch.equal(y16.cpu(), want.half())
+
+
+@pytest.mark.parametrize("H,I,E,k,xdt,renorm", [
+    (128, 128, 4, 2, "float32", False), (640, 384, 17, 3, "float16", True), (2048, 768, 128, 8, "float32", True),
+    (1152, 1152, 9, 9, "float32", False),          # every expert takes every token
+    (4096, 256, 1024, 64, "float16", False)])      # the most experts, slots and columns
+def test_moe_one_or_two_tokens_equal_general_path(env, H, I, E, k, xdt, renorm):
+    """One or two tokens take kernels of their own; a token's output does not
+    depend on the others, so each must equal, bit for bit, its row of a 6-token
+    call, which takes the general path (and whose results the oracle tests
+    hold)."""
+    torch, ops, d = env
+    _say(f"moe one or two tokens H={H} I={I} E={E} k={k}")
+    g = torch.Generator(device=d).manual_seed(H + E)
+    T = 6
+    x = torch.randn((T, H), generator=g, device=d).to(getattr(torch, xdt))
+    x[3] = 0                                        # zero rows quantize with scale 1
+    logits = torch.randn((T, E), generator=g, device=d)
+    logits[5] = 0.25                                # ties: the lowest experts
+    wg = torch.randint(-127, 128, (E, 2 * I, H), generator=g, device=d, dtype=torch.int8)
+    wd = torch.randint(-127, 128, (E, H, I), generator=g, device=d, dtype=torch.int8)
+    sg = torch.rand((E, 2 * I), generator=g, device=d) * 0.002
+    sd = torch.rand((E, H), generator=g, device=d) * 0.002
+    for odt in (torch.float32, torch.float16):
+        full = torch.full((T, H), float("nan"), device=d, dtype=odt)
+        sync(torch)
+        ops.moe_w8a8(x, logits, wg, sg, wd, sd, full, T, H, I, E, k, renorm)
+        for t, n in ((0, 1), (3, 1), (1, 2), (2, 2), (4, 2)):
+            out = torch.full((n, H), float("nan"), device=d, dtype=odt)
+            sync(torch)
+            ops.moe_w8a8(x[t:t + n], logits[t:t + n].contiguous(), wg, sg, wd, sd, out, n, H, I, E, k, renorm)
+            sync(torch)
+            assert torch.equal(out, full[t:t + n]), (t, n, odt)
