@@ -80,7 +80,10 @@ __device__ __forceinline__ void route_token(const float* __restrict__ lr, float*
     // retired by setting them to -inf (probabilities are >= 0). Each lane's
     // best (strict '>' over ascending e: its lowest index among equals), then
     // the wave max and the lowest index holding it, both as DPP reductions
-    // (no LDS-queue shuffles in the dependent chain).
+    // (no LDS-queue shuffles in the dependent chain). Logits with a NaN or +inf,
+    // or only -inf, make every probability NaN, and no comparison finds one: the
+    // ids are then 0 .. top_k - 1 and the weights NaN, as what follows indexes
+    // memory with the ids.
     float wsum = 0.f;
     float myw = 0.f;
     int myid = 0;
@@ -91,8 +94,12 @@ __device__ __forceinline__ void route_token(const float* __restrict__ lr, float*
             const float v = p[e];
             if (v > bv) { bv = v; bi = e; }
         }
-        const float m = wmax(bv);
-        const int mi = wmin_i(bv == m ? bi : 0x7fffffff);
+        float m = wmax(bv);
+        int mi = wmin_i(bv == m ? bi : 0x7fffffff);
+        if (mi >= E) {
+            m = NAN;
+            mi = kk;
+        }
         if (lane == kk) { myw = m; myid = mi; }
         wsum += m;
         if (lane == (mi & 63)) p[mi] = -INFINITY;

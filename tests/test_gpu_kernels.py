@@ -896,3 +896,41 @@ def test_moe_one_or_two_tokens_equal_general_path(env, H, I, E, k, xdt, renorm):
             ops.moe_w8a8(x[t:t + n], logits[t:t + n].contiguous(), wg, sg, wd, sd, out, n, H, I, E, k, renorm)
             sync(torch)
             assert torch.equal(out, full[t:t + n]), (t, n, odt)
+
+
+@pytest.mark.parametrize("T", [1, 2, 6])
+def test_moe_logits_without_an_order(env, T):
+    """Logits with a NaN or an inf, or only -inf, give NaN probabilities: the
+    token gets valid, distinct experts and a NaN output, the others their own."""
+    torch, ops, d = env
+    H, I, E, k = 128, 128, 9, 3
+    g = torch.Generator(device=d).manual_seed(T)
+    x = torch.randn((T, H), generator=g, device=d)
+    logits = torch.randn((T, E), generator=g, device=d)
+    wg = torch.randint(-127, 128, (E, 2 * I, H), generator=g, device=d, dtype=torch.int8)
+    wd = torch.randint(-127, 128, (E, H, I), generator=g, device=d, dtype=torch.int8)
+    sg = torch.rand((E, 2 * I), generator=g, device=d) * 0.01
+    sd = torch.rand((E, H), generator=g, device=d) * 0.01
+
+    def layer(lg, renorm):
+        out = torch.empty((T, H), device=d)
+        ops.moe_w8a8(x, lg, wg, sg, wd, sd, out, T, H, I, E, k, renorm)
+        torch.cuda.synchronize()
+        return out
+
+    for bad in (float("nan"), float("inf"), None):
+        lg = logits.clone()
+        if bad is None:
+            lg[T - 1] = float("-inf")
+        else:
+            lg[T - 1, 4] = bad
+        _say(f"moe logits without an order T={T} {bad}")
+        w = torch.empty((T, k), device=d)
+        ids = torch.empty((T, k), device=d, dtype=torch.int32)
+        ops.moe_route(lg, w, ids, T, E, k, True)
+        torch.cuda.synchronize()
+        assert ids[T - 1].tolist() == list(range(k)) and torch.isnan(w[T - 1]).all()
+        for renorm in (False, True):
+            out, want = layer(lg, renorm), layer(logits, renorm)
+            assert torch.isnan(out[T - 1]).all()
+            assert torch.equal(out[:T - 1], want[:T - 1])
