@@ -30,6 +30,8 @@ namespace pio {
 
 int gemm_w8_planes(const int8_t* xp, const int8_t* w, const float* s_w, const float* bias, float* y, int64_t ldy, int M,
                    int N, int K, bool resid, Scratch& ws, const float** part, int* splits, hipStream_t st);
+int gemm_w8_planes_swiglu(const int8_t* xp, const int8_t* w, const float* s_w, int8_t* act, int M, int I, int K, bool* done,
+                          hipStream_t st);
 
 // x[m] = embed[ids[pos0 + m]] (an out-of-range id reads row 0, as the step).
 __global__ __launch_bounds__(256) void pf_embed_kernel(const float* __restrict__ embed, const int32_t* __restrict__ ids,
@@ -155,7 +157,6 @@ __global__ __launch_bounds__(64) void pf_qkv_finish_kernel(const float* __restri
 // act[m][i] = silu(g) * u into the planes of act, 4 channels per thread, row m =
 // wf_row_of_block(blockIdx.y). part: g and u are the gate_up linear's K slices,
 // formed as the GEMM's reduce forms them (no bias); else the rows of gu.
-__device__ __forceinline__ float pf_silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 __global__ __launch_bounds__(256) void pf_swiglu_kernel(const float* __restrict__ gu, const float* __restrict__ part,
                                                         int splits, int M, int I, const float* __restrict__ s_w,
                                                         int8_t* __restrict__ act) {
@@ -178,8 +179,8 @@ __global__ __launch_bounds__(256) void pf_swiglu_kernel(const float* __restrict_
         g = *(const float4*)(gu + r);
         u = *(const float4*)(gu + r + I);
     }
-    wf_put4(act, m, i, I, make_float4(pf_silu_mul(g.x, u.x), pf_silu_mul(g.y, u.y), pf_silu_mul(g.z, u.z),
-                                      pf_silu_mul(g.w, u.w)));
+    wf_put4(act, m, i, I, make_float4(wf_silu_mul(g.x, u.x), wf_silu_mul(g.y, u.y), wf_silu_mul(g.z, u.z),
+                                      wf_silu_mul(g.w, u.w)));
 }
 
 // A residual linear's K slices finished into x (x += slices * s, as the
@@ -322,12 +323,18 @@ int prefill(Qwen3Dec* d, int M, bool logits) {
             PIO_LAUNCHED();
         }
         {
-            Scratch pw;
-            const float* part;
-            int sp;
-            PIO_TRY(gemm_w8_planes(h, L.w_gu, L.s_gu, nullptr, gu, 2 * I, M, 2 * I, H, false, pw, &part, &sp, st));
-            pf_swiglu_kernel<<<dim3(ceil_div(I, 1024), rb), 256, 0, st>>>(gu, sp ? part : nullptr, sp, M, I, L.s_gu, act);
-            PIO_LAUNCHED();
+            bool fused;
+            PIO_TRY(gemm_w8_planes_swiglu(h, L.w_gu, L.s_gu, act, M, I, H, &fused, st));
+            if (!fused) {
+                Scratch pw;
+                const float* part;
+                int sp;
+                PIO_TRY(gemm_w8_planes(h, L.w_gu, L.s_gu, nullptr, gu, 2 * I, M, 2 * I, H, false, pw, &part, &sp,
+                                       st));
+                pf_swiglu_kernel<<<dim3(ceil_div(I, 1024), rb), 256, 0, st>>>(gu, sp ? part : nullptr, sp, M, I,
+                                                                                  L.s_gu, act);
+                PIO_LAUNCHED();
+            }
         }
         {
             Scratch pw;

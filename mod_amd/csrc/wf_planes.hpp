@@ -35,6 +35,9 @@ __device__ __forceinline__ void wf_split3_pair(float a, float c, int& h, int& m,
     l = (int)__builtin_amdgcn_perm(__float_as_uint(c2), __float_as_uint(a2), 0x07060302u);
 }
 
+// SwiGLU of the prompt's MLP.
+__device__ __forceinline__ float wf_silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
+
 // Values k .. k + 3 of row m (k % 4 == 0) into the planes of a [..][K] matrix.
 __device__ __forceinline__ void wf_put4(int8_t* planes, int m, int k, int K, float4 v) {
     int2 h, d, l;

@@ -77,6 +77,31 @@ def test_prefill_last_logits_and_chunks(torch_dev, kv_dtype):
     assert diff <= (1e-4 if kv_dtype == "float32" else 2e-3), diff
 
 
+@pytest.mark.parametrize("P,intermediate", [(385, 3072), (421, 3136), (512, 3072)])
+def test_prefill_long_batch(torch_dev, P, intermediate):
+    """From 385 rows the gate_up GEMM's epilogue forms silu(g) * u (row tiles of
+    1, 37 and 128 rows at the end): logits against the oracle, and against the
+    same prompt in batches of at most 100, whose SwiGLU is a kernel of its own
+    (the bar of the test above: fp32 rounding in another order)."""
+    from mod_amd.qwen3 import Qwen3Int8Decoder, random_weights
+    cfg, rcfg = _small(max_seq=512, intermediate=intermediate)
+    w = random_weights(cfg, seed=63)
+    dec = Qwen3Int8Decoder(cfg, w)
+    prompt = np.random.default_rng(64).integers(0, cfg.vocab, size=P).astype(np.int32)
+    _say(f"prefill long batch P={P} I={intermediate}")
+    dec.reset(prompt)
+    dec.prefill(P, logits=True)
+    one = dec.read(0, with_logits=True)[1].copy()
+    _against_oracle(one[None], prompt, [P - 1], rcfg, w, f"prefill of {P}")
+    dec.reset(prompt)
+    for a in range(0, P, 100):
+        dec.prefill(min(100, P - a), logits=a + 100 >= P)
+    parts = dec.read(0, with_logits=True)[1]
+    diff = float(np.abs(parts - one).max()) / float(np.sqrt(np.mean(one.astype(np.float64) ** 2)))
+    _say(f"one batch vs parts: max diff {diff:.2e} x rms")
+    assert diff <= 1e-4, diff
+
+
 def test_prefill_refuses_generated_positions(torch_dev):
     from mod_amd.ops import RocmError
     from mod_amd.qwen3 import Qwen3Int8Decoder, random_weights
