@@ -277,6 +277,7 @@ struct GroupedParams {
     unsigned* amax;           // SwiGLU: per position, max |h| as float bits (zeroed beforehand)
     int64_t a_bytes;          // extent of A (< 2^31: rows past a tile's count read as zeros)
     int N, K;
+    const int32_t* active;    // [0] experts with tokens, then their ids; or nullptr: block y is expert y
 };
 
 // Block (n-tile, expert) on the register-staged v6 engine (the expert layer
@@ -302,7 +303,11 @@ __device__ __forceinline__ float silu_mul(float g, float u) {
 template <int NK, bool SWIGLU>
 __global__ __launch_bounds__(MOE_THREADS, 2) void moe_grouped_gemm_kernel(GroupedParams p) {
     extern __shared__ __attribute__((aligned(16))) int8_t lds_moe[];
-    const int e = blockIdx.y;
+    int e = blockIdx.y;
+    if (p.active) {
+        if (e >= p.active[0]) return;
+        e = p.active[1 + e];
+    }
     // n0: first weight row of the tile; SwiGLU tiles take 64 gate + 64 up rows
     const int n0 = SWIGLU ? blockIdx.x * (MoeTile::BN / 2) : blockIdx.x * MoeTile::BN;
     const int I = p.N / 2;
@@ -418,10 +423,16 @@ static void launch_grouped(const GroupedParams& g, dim3 grid, int nk, hipStream_
 // integer sums, scales and order as above, so the same bits.
 // Qwen3-30B-A3B layer: T = 1 36.4 -> 25.2 us. From T = 3 the path above is the
 // faster one (41 / 46 us at 3, 86 / 114 at 16): these loads cover half a line of
-// a row each and stream at 4 TB/s, its tiles at 4.6 and up, and one block takes
-// longer to route many tokens than the launch it saves.
+// a row each and stream at 4 TB/s, its tiles at 4.6 and up.
 constexpr int MS_MAX_T = 2;        // tokens (and rows of an expert)
-constexpr int MS_MAX_P = 64 * MS_MAX_T;   // (token, slot) pairs
+// Tokens up to which the front kernel replaces the route and group launches:
+// one round of its 16 waves, a wave per job. Above MS_MAX_T the GEMMs are the
+// general ones, on blocks for the listed experts only: T = 4 / 5 / 8 of the same
+// layer 47.7 / 52.6 / 65.3 -> 45.1 / 49.6 / 63.0 us. T = 3 was slower in each of two
+// runs (41.4 -> 42.7 us, cause not found) and keeps the general path.
+constexpr int FR_MAX_T = 8;
+constexpr int FR_MAX_P = 64 * FR_MAX_T;   // (token, slot) pairs
+static bool front_path(int T) { return T <= MS_MAX_T || (T > 3 && T <= FR_MAX_T); }
 constexpr int MS_SET = 512;        // K values of a wave's rows per register set
 constexpr int MS_LOADS = MS_SET / 64;
 
@@ -441,7 +452,7 @@ struct MoeFront {
 template <typename XT>
 __global__ __launch_bounds__(1024) void moe_front_kernel(MoeFront p) {
     extern __shared__ float fr_p[];               // [T][E] probabilities
-    __shared__ __attribute__((aligned(16))) int32_t ids[MS_MAX_P];
+    __shared__ __attribute__((aligned(16))) int32_t ids[FR_MAX_P];
     __shared__ int32_t off[ROUTE_MAX_E];
     __shared__ int wsum_[16];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, P = p.T * p.top_k;
@@ -704,7 +715,7 @@ struct MoeWs {
     int32_t* offsets;
     int32_t* row_token;
     int32_t* pos_of_pair;
-    int32_t* active;     // [1 + MS_MAX_P], the path of one or two tokens
+    int32_t* active;     // [1 + FR_MAX_P], calls of few tokens
     int8_t* qx;
     float* sx;
     float* h;            // [P][I] SwiGLU output (fp32)
@@ -727,7 +738,7 @@ static MoeWs moe_layout(char* base, int T, int H, int I, int E, int k) {
     w.offsets = (int32_t*)take((size_t)(E + 1) * 4);
     w.row_token = (int32_t*)take(P * 4);
     w.pos_of_pair = (int32_t*)take(P * 4);
-    w.active = (int32_t*)take((size_t)(MS_MAX_P + 1) * 4);
+    w.active = (int32_t*)take((size_t)(FR_MAX_P + 1) * 4);
     w.qx = (int8_t*)take((size_t)T * H);
     w.sx = (float*)take((size_t)T * 4);
     w.h = (float*)take(P * I * 4);
@@ -787,14 +798,28 @@ int moe_w8a8(const void* x, int x_dtype, const float* logits, const int8_t* w_gu
         PIO_LAUNCHED();
         return PIO_OK;
     };
-    if (T <= MS_MAX_T) {
+    const bool front = front_path(T);
+    if (front) {
         MoeFront f{logits, x, H, T, E, top_k, renorm, w.topk_w, w.topk_id, w.qx, w.sx, w.amax, w.offsets, w.row_token,
                    w.pos_of_pair, w.active};
         const size_t lds = (size_t)T * E * sizeof(float);
         if (x_dtype == PIO_F32) moe_front_kernel<float><<<1, 1024, lds, st>>>(f);
         else moe_front_kernel<_Float16><<<1, 1024, lds, st>>>(f);
         PIO_LAUNCHED();
-        const int na = std::min(E, P);
+    } else {
+        if (x_dtype == PIO_F32)
+            moe_route_quant_kernel<float><<<ceil_div(T, 2), 256, 0, st>>>(
+                logits, (const float*)x, H, w.topk_w, w.topk_id, w.qx, w.sx, T, E, top_k, renorm, w.amax);
+        else
+            moe_route_quant_kernel<_Float16><<<ceil_div(T, 2), 256, 0, st>>>(
+                logits, (const _Float16*)x, H, w.topk_w, w.topk_id, w.qx, w.sx, T, E, top_k, renorm, w.amax);
+        PIO_LAUNCHED();
+        moe_group_kernel<<<E, 512, 0, st>>>(w.topk_id, T, E, top_k, w.offsets, w.row_token,
+                                            w.pos_of_pair);
+        PIO_LAUNCHED();
+    }
+    const int na = front ? std::min(E, P) : E;   // experts that may have tokens
+    if (T <= MS_MAX_T) {
         MoeSmall g{w.active, w.offsets, w.row_token, w.qx, w.sx, nullptr, w.amax, w_gu, s_gu, w.h, 2 * I, H};
         PIO_TRY((launch_small<true, 1>(g, dim3(I / 16, na), ceil_div(H, MS_SET), st)));
         MoeSmall d{w.active, w.offsets, w.row_token, nullptr, nullptr, w.h, w.amax, w_down, s_down, w.d, H, I};
@@ -802,22 +827,12 @@ int moe_w8a8(const void* x, int x_dtype, const float* logits, const int8_t* w_gu
         return combine();
     }
 
-    if (x_dtype == PIO_F32)
-        moe_route_quant_kernel<float><<<ceil_div(T, 2), 256, 0, st>>>(
-            logits, (const float*)x, H, w.topk_w, w.topk_id, w.qx, w.sx, T, E, top_k, renorm, w.amax);
-    else
-        moe_route_quant_kernel<_Float16><<<ceil_div(T, 2), 256, 0, st>>>(
-            logits, (const _Float16*)x, H, w.topk_w, w.topk_id, w.qx, w.sx, T, E, top_k, renorm, w.amax);
-    PIO_LAUNCHED();
-    moe_group_kernel<<<E, 512, 0, st>>>(w.topk_id, T, E, top_k, w.offsets, w.row_token,
-                                        w.pos_of_pair);
-    PIO_LAUNCHED();
-
     GroupedParams g{};
     g.A = w.qx; g.a_rows = w.row_token; g.s_a = w.sx;
     g.W = w_gu; g.s_w = s_gu; g.offsets = w.offsets; g.C = w.h; g.amax = w.amax;
     g.N = 2 * I; g.K = H; g.a_bytes = (int64_t)T * H;
-    launch_grouped<1, true>(g, dim3(I / (MoeTile::BN / 2), E), H / 128, st);
+    g.active = front ? w.active : nullptr;
+    launch_grouped<1, true>(g, dim3(I / (MoeTile::BN / 2), na), H / 128, st);
     PIO_LAUNCHED();
 
     moe_requant_kernel<<<ceil_div(P, 4), 256, 0, st>>>(w.h, w.amax, w.qh, w.sh, P, I);
@@ -827,7 +842,8 @@ int moe_w8a8(const void* x, int x_dtype, const float* logits, const int8_t* w_gu
     d.A = w.qh; d.a_rows = nullptr; d.s_a = w.sh;
     d.W = w_down; d.s_w = s_down; d.offsets = w.offsets; d.C = w.d;
     d.N = H; d.K = I; d.a_bytes = (int64_t)P * I;
-    launch_grouped<1, false>(d, dim3(ceil_div(H, MoeTile::BN), E), I / 128, st);
+    d.active = g.active;
+    launch_grouped<1, false>(d, dim3(ceil_div(H, MoeTile::BN), na), I / 128, st);
     PIO_LAUNCHED();
 
     return combine();

@@ -934,3 +934,33 @@ def test_moe_logits_without_an_order(env, T):
             out, want = layer(lg, renorm), layer(logits, renorm)
             assert torch.isnan(out[T - 1]).all()
             assert torch.equal(out[:T - 1], want[:T - 1])
+
+
+@pytest.mark.parametrize("H,I,E,k,xdt", [
+    (128, 128, 4, 2, "float32"), (640, 384, 17, 3, "float16"), (2048, 768, 128, 8, "float32"),
+    (1152, 1152, 9, 9, "float32"),                 # every expert takes every token
+    (256, 256, 1024, 64, "float16")])              # the most experts and slots
+def test_moe_few_tokens_equal_general_path(env, H, I, E, k, xdt):
+    """4 to 8 tokens are routed and grouped by one block, and only the experts
+    it lists get GEMM blocks: each call must equal, bit for bit, its rows of a
+    12-token call, which the general path takes."""
+    torch, ops, d = env
+    _say(f"moe few tokens H={H} I={I} E={E} k={k}")
+    g = torch.Generator(device=d).manual_seed(H + E)
+    T = 12
+    x = torch.randn((T, H), generator=g, device=d).to(getattr(torch, xdt))
+    logits = torch.randn((T, E), generator=g, device=d)
+    logits[4:6] = 0.25                              # ties: the lowest experts
+    wg = torch.randint(-127, 128, (E, 2 * I, H), generator=g, device=d, dtype=torch.int8)
+    wd = torch.randint(-127, 128, (E, H, I), generator=g, device=d, dtype=torch.int8)
+    sg = torch.rand((E, 2 * I), generator=g, device=d) * 0.002
+    sd = torch.rand((E, H), generator=g, device=d) * 0.002
+    full = torch.full((T, H), float("nan"), device=d)
+    sync(torch)
+    ops.moe_w8a8(x, logits, wg, sg, wd, sd, full, T, H, I, E, k, True)
+    for t, n in ((0, 3), (3, 4), (4, 7), (2, 8), (4, 8)):
+        out = torch.full((n, H), float("nan"), device=d)
+        sync(torch)
+        ops.moe_w8a8(x[t:t + n], logits[t:t + n].contiguous(), wg, sg, wd, sd, out, n, H, I, E, k, True)
+        sync(torch)
+        assert torch.equal(out, full[t:t + n]), (t, n)
