@@ -602,8 +602,15 @@ static int run_w8p_tiles(W8pParams p, int blocks, int min_steps, Scratch* ws, co
     p.n_tiles = ceil_div(p.N, 32 * TN * (4 / WM));
     const int tiles = p.m_tiles * p.n_tiles;
     p.per_xcd = ceil_div(tiles, 8);
-    int splits = wf_splits(tiles, p.K, 64, blocks, min_steps);
-    p.ks = ceil_div(ceil_div(p.K, 64), splits) * 64;
+    const int steps = ceil_div(p.K, 64);
+    // Few rows, many tiles: as many slices as fill the blocks, not a power of two
+    // (96 tiles: 5 slices, 480 blocks, against 4 that give half the CUs two blocks
+    // and half one: (13, 12288, 4096) 24.7 -> 22.6 us, (32, 12288, 2064) 21.4 -> 20.3).
+    // At 64 tiles and fewer the powers of two fill them as well with fewer
+    // partials ((32, 5003, 4096), 40 tiles: 18.55 us against 18.65).
+    int splits = WM > 1 || tiles <= 64 ? wf_splits(tiles, p.K, 64, blocks, min_steps)
+                                       : std::max(1, std::min(blocks / tiles, steps / min_steps));
+    p.ks = ceil_div(steps, splits) * 64;
     splits = ceil_div(p.K, p.ks);
     if (splits == 1) return launch_w8p<YT, RESID ? WF_RESID : WF_STORE, WM, TN>(p, 1, st);
     YT* y = (YT*)p.y;
