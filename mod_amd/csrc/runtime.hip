@@ -143,6 +143,20 @@ static void empty_cache_locked(Alloc& a) {
     a.free_lists.clear();
 }
 
+// hipMalloc and hipFree are refused, and end the capture, while any stream
+// captures in the global mode (torch.cuda.graph's default) or one of this
+// thread in the thread-local mode. Neither touches the capturing stream, so the
+// allocator makes its calls in the relaxed mode: an op's first call, with its
+// workspace not yet in the cache, can be the captured one.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { swap(); }
+    ~RelaxedCapture() { swap(); }
+    void swap() {
+        if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) (void)hipGetLastError();
+    }
+};
+
 int device_alloc(void** out, size_t bytes, hipStream_t stream) {
     *out = nullptr;
     int dev = 0;
@@ -189,6 +203,7 @@ int device_alloc(void** out, size_t bytes, hipStream_t stream) {
         a.cached -= r;
     } else {
         void* p = nullptr;
+        RelaxedCapture relaxed;
         hipError_t e = hipMalloc(&p, r);
         if (e != hipSuccess) {
             (void)hipGetLastError();

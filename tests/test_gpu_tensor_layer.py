@@ -13,11 +13,13 @@ create_tensor_typed, against the oracle:
 * the allocator around graph capture (begin_capture / end_capture /
   replay_graph, backend.py:801-810): a workspace an op frees while its stream
   captures stays with the graph, so a tensor allocated afterwards cannot alias
-  it; destroy_stream releases what is cached for the stream;
+  it; an op's first call can be the captured one; destroy_stream releases what
+  is cached for the stream;
 * the arena (init_memory_pool / reset_memory_pool, tensor_ops.c:74-93) and a
   clean process exit after the persistent decoder, in a child process (the
   arena changes where every later tensor of a process lives).
 """
+import ctypes
 import os
 import subprocess
 import sys
@@ -296,6 +298,69 @@ def test_torch_graph_of_several_ops_with_workspaces(torch_dev):
             assert torch.equal(y, e), f"replay {r}, output {i}"
         junk = torch.randn(1 << 20, device=d) * 2   # eager work between replays
         del junk
+
+
+@pytest.mark.parametrize("op", ["attention", "w8"])
+def test_first_call_inside_a_global_mode_capture(torch_dev, op):
+    """The first call of an op on a stream, with its workspace not in the cache,
+    captured by torch.cuda.graph (whose default mode forbids allocation calls
+    that could touch a capturing stream): attention with its keys split over
+    workgroups, and an fp32 W8 linear that splits its activations first. Every
+    replay gives the eager result."""
+    import torch
+    from mod_amd import backend as B, ops
+    from mod_amd.ops import lib, check
+    d = torch_dev
+    g = torch.Generator(device=d).manual_seed(3)
+    st = torch.cuda.Stream()
+    if op == "attention":
+        q, k, v = (torch.randn(s, generator=g, device=d) for s in ((2, 1, 4, 128), (2, 1500, 2, 128), (2, 1500, 2, 128)))
+        tq, tk, tv = (B.Tensor.from_numpy(t.cpu().numpy()) for t in (q, k, v))
+        out = B.Tensor([2, 1, 4, 128])
+
+        def call():
+            check(lib.tensor_scaled_dot_product_attention_status(tq._handle, tk._handle, tv._handle, out._handle,
+                                                                 ctypes.c_float(0.1)))
+
+        def result():
+            return out.numpy().copy()
+
+        def clear():
+            out.fill(0.0)
+    else:
+        M, N, K = 64, 4096, 4096
+        x, s = torch.randn((M, K), generator=g, device=d), torch.rand(N, generator=g, device=d)
+        w = torch.randint(-127, 128, (N, K), generator=g, device=d, dtype=torch.int8)
+        y = torch.empty((M, N), device=d)
+
+        def call():
+            ops.gemv_w8(x, w, s, None, y, M, N, K)
+
+        def result():
+            return y.cpu().numpy()
+
+        def clear():
+            y.zero_()
+    torch.cuda.synchronize()
+    _say(f"first call inside a capture: {op}")
+    call()
+    B.synchronize()
+    want = result()
+    lib.tensor_empty_cache()
+    graph = torch.cuda.CUDAGraph()
+    lib.set_current_stream(st.cuda_stream)
+    try:
+        with torch.cuda.graph(graph, stream=st):
+            call()
+    finally:
+        lib.set_current_stream(None)
+    for r in range(3):
+        clear()
+        B.synchronize()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(result(), want), f"replay {r}"
 
 
 def test_destroy_stream_releases_its_cache(T):
