@@ -38,6 +38,7 @@
 
 #include <algorithm>
 #include <float.h>
+#include <type_traits>
 
 namespace pio {
 
@@ -94,6 +95,66 @@ __device__ __forceinline__ void at_store(const AttnArgs& a, int D, int b, int s,
     } else {
         *(at_f4*)(a.out + b * a.o_b + (int64_t)s * a.o_s + hd * D + sl) = v;
     }
+}
+
+// A finished column's 4 slots from sl: v, the sum of exp(score - m) v, over l, the
+// sum of the weights; D / 4 consecutive lanes have one column. The sum can leave
+// the fp32 range where softmax(s) v does not (T keys with |v| above FLT_MAX / T),
+// so a column with an inf or NaN among its outputs whose scores are in order
+// (0 < l < inf) is formed again by its lanes alone, as softmax(s) v is written:
+// the weights' sum, then normalised weights times v.
+template <int D, typename KT, bool CAUSAL>
+__device__ __forceinline__ at_f4 at_finish(const AttnArgs& a, int b, int g, int s, int hd, int sl, at_f4 v, float m,
+                                           float l) {
+    constexpr bool PAIR = sizeof(KT) == 2;
+    constexpr int U = 4;                   // keys at a time
+    const at_f4 r = v * (1.0f / l);
+    bool odd = false;
+#pragma unroll
+    for (int j = 0; j < 4; j++) odd |= !(fabsf(r[j]) <= FLT_MAX);
+    constexpr unsigned long long group = (1ull << (D / 4)) - 1;
+    if (CAUSAL || !(__ballot(odd) >> (threadIdx.x & 63 & ~(D / 4 - 1)) & group) || !(l > 0.f && l <= FLT_MAX)) return r;
+    const int limit = CAUSAL ? a.pos0 + s + 1 : a.T;
+    const float* qr = a.q + b * a.q_b + (int64_t)s * a.q_s + hd * D;
+    const KT* kb = (const KT*)a.k + b * a.kv_b + g * a.kv_h + sl;
+    const KT* vb = (const KT*)a.v + b * a.kv_b + g * a.kv_h + sl;
+    float q[4], inv = 1.f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) q[j] = qr[at_dim<PAIR>(sl + j)];
+    for (int pass = 0; pass < 2; pass++) {
+        float sum = 0.f;
+        at_f4 o = {0.f, 0.f, 0.f, 0.f};
+        for (int t0 = 0; t0 < limit; t0 += U) {
+            float e[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const KT* kr = kb + (int64_t)min(t0 + u, limit - 1) * a.kv_t;
+                e[u] = 0.f;
+#pragma unroll
+                for (int j = 0; j < 4; j++) e[u] = fmaf(q[j], (float)kr[j], e[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+#pragma unroll
+                for (int x = D / 8; x >= 1; x >>= 1) e[u] += __shfl_xor(e[u], x, 64);
+                e[u] = expf(e[u] * a.scale - m);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (t0 + u >= limit) break;
+                if (pass == 0) {
+                    sum += e[u];
+                } else {
+                    const KT* vr = vb + (int64_t)(t0 + u) * a.kv_t;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) o[j] = fmaf(e[u] * inv, (float)vr[j], o[j]);
+                }
+            }
+        }
+        if (pass) return o;
+        inv = 1.0f / sum;
+    }
+    return r;
 }
 
 template <int D, typename KT, bool CAUSAL>
@@ -325,9 +386,8 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams 
             }
             continue;
         }
-        const float inv = 1.0f / cl;
         const int s = (c0 + c) / p.G, hd = g * p.G + (c0 + c) - s * p.G;
-        at_store<PAIR, CAUSAL>(a, D, b, s, hd, sl, v * inv);
+        at_store<PAIR, CAUSAL>(a, D, b, s, hd, sl, at_finish<D, KT, CAUSAL>(a, b, g, s, hd, sl, v, cm, cl));
     }
 }
 
@@ -484,7 +544,8 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_vec_kernel(AttnParams p
                 p.part_ml[2 * at + 1] = cl;
             }
         } else {
-            at_store<false, false>(a, D, b, s, g * p.G + c - s * p.G, sl, v * (1.0f / cl));
+            const int hd = g * p.G + c - s * p.G;
+            at_store<false, false>(a, D, b, s, hd, sl, at_finish<D, float, false>(a, b, g, s, hd, sl, v, cm, cl));
         }
     }
 }
@@ -530,8 +591,9 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
         l += sl_[z] * f;
         v += *(const at_f4*)&so[z][sl] * f;
     }
-    const int s = c / p.G;
-    at_store<PAIR, CAUSAL>(a, D, b, s, g * p.G + c - s * p.G, sl, v * (1.0f / l));
+    const int s = c / p.G, hd = g * p.G + c - s * p.G;
+    typedef typename std::conditional<PAIR, _Float16, float>::type KT;
+    at_store<PAIR, CAUSAL>(a, D, b, s, hd, sl, at_finish<D, KT, CAUSAL>(a, b, g, s, hd, sl, v, mx, l));
 }
 
 bool attn_mfma_supported(const AttnArgs& a) {

@@ -168,6 +168,42 @@ def test_attention_tiles(B, Bn, S, H, Hk, T, D):
     assert np.isfinite(np.delete(got, 3, axis=-1)).all()
 
 
+@pytest.mark.parametrize("Bn,S,H,Hk,T,D", [
+    (1, 33, 4, 2, 64, 128), (1, 40, 3, 1, 61, 64),       # tiles of 32 columns, keys unsplit
+    (1, 20, 4, 2, 1501, 128), (2, 9, 16, 2, 777, 64),    # keys split over workgroups
+    (1, 2, 2, 1, 97, 64), (1, 1, 8, 2, 100, 128),        # 2 and 4 columns per kv head: the VALU kernel
+    (2, 1, 4, 2, 1500, 128), (3, 1, 2, 2, 2048, 64)])
+def test_attention_value_range(B, Bn, S, H, Hk, T, D):
+    """softmax(s) v is finite for finite v, also where a sum of exp(s - max) v
+    is not: values up to 3e38 in one kv head, out of place and into q, within
+    the bar of the other tests; beside them a query of NaN, whose own rows alone
+    are NaN."""
+    from mod_amd import ops
+    from mod_amd.ops import lib
+    _say(f"attention value range B{Bn} S{S} H{H} Hk{Hk} T{T} D{D}")
+    rng = np.random.default_rng(S * 11 + T)
+    q = rng.standard_normal((Bn, S, H, D)).astype(np.float32)
+    k = rng.standard_normal((Bn, T, Hk, D)).astype(np.float32)
+    v = rng.standard_normal((Bn, T, Hk, D)).astype(np.float32)
+    v[..., 0, :] = rng.uniform(-3e38, 3e38, (Bn, T, D))
+    v[..., 0, 0], v[..., 0, D - 1] = 3e38, -3e38
+    q[Bn - 1, S - 1, H - 1, 5] = np.nan
+    want = mo.sdpa(q, k, v, 1 / np.sqrt(D))
+    tq, tk, tv = _t(B, q), _t(B, k), _t(B, v)
+    got = B.scaled_dot_product_attention(tq, tk, tv).numpy()
+    bad = np.zeros((Bn, S, H), bool)
+    bad[Bn - 1, S - 1, H - 1] = True
+    assert np.isnan(got[bad]).all() and np.isfinite(got[~bad]).all()
+    rep = H // Hk
+    for h in range(H):
+        vmax = float(np.abs(v[:, :, h // rep]).max())
+        d = np.abs(got[:, :, h].astype(np.float64) - want[:, :, h])[~bad[:, :, h]]
+        assert d.size == 0 or float(d.max()) <= RTOL * vmax, h
+    assert lib.tensor_scaled_dot_product_attention_status(tq._handle, tk._handle, tv._handle, tq._handle,
+                                                          ctypes.c_float(1 / np.sqrt(D))) == ops.OK
+    assert np.array_equal(tq.numpy(), got, equal_nan=True)
+
+
 def test_slice_set_slice_cat_reshape_exact(B):
     rng = np.random.default_rng(5)
     x = rng.standard_normal((3, 9, 4, 8)).astype(np.float32)
