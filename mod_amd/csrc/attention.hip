@@ -102,7 +102,9 @@ __device__ __forceinline__ void at_store(const AttnArgs& a, int D, int b, int s,
 // the fp32 range where softmax(s) v does not (T keys with |v| above FLT_MAX / T),
 // so a column with an inf or NaN among its outputs whose scores are in order
 // (0 < l < inf) is formed again by its lanes alone, as softmax(s) v is written:
-// the weights' sum, then normalised weights times v.
+// the weights' sum, then normalised weights times v, over the keys that the column
+// sees. (In a causal tile an inf or NaN in the value row of a later key meets the
+// zero weights of earlier columns and makes them NaN: they come out right here.)
 template <int D, typename KT, bool CAUSAL>
 __device__ __forceinline__ at_f4 at_finish(const AttnArgs& a, int b, int g, int s, int hd, int sl, at_f4 v, float m,
                                            float l) {
@@ -113,7 +115,7 @@ __device__ __forceinline__ at_f4 at_finish(const AttnArgs& a, int b, int g, int 
 #pragma unroll
     for (int j = 0; j < 4; j++) odd |= !(fabsf(r[j]) <= FLT_MAX);
     constexpr unsigned long long group = (1ull << (D / 4)) - 1;
-    if (CAUSAL || !(__ballot(odd) >> (threadIdx.x & 63 & ~(D / 4 - 1)) & group) || !(l > 0.f && l <= FLT_MAX)) return r;
+    if (!(__ballot(odd) >> (threadIdx.x & 63 & ~(D / 4 - 1)) & group) || !(l > 0.f && l <= FLT_MAX)) return r;
     const int limit = CAUSAL ? a.pos0 + s + 1 : a.T;
     const float* qr = a.q + b * a.q_b + (int64_t)s * a.q_s + hd * D;
     const KT* kb = (const KT*)a.k + b * a.kv_b + g * a.kv_h + sl;
@@ -321,7 +323,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams 
         m = mt;
         // a key past the last one: its weight is zero, and what is read in its
         // place must not be inf or NaN. (A causal tile's later keys are rows of
-        // this batch: an inf there also meets zero weights of earlier columns.)
+        // this batch: see at_finish.)
         auto zero_v = [&](int e) {
             if (edge && t0 + 8 * (e >> 2) + 4 * h + (e & 3) >= limit_all)
 #pragma unroll

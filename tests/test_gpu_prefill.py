@@ -102,6 +102,63 @@ def test_prefill_long_batch(torch_dev, P, intermediate):
     assert diff <= 1e-4, diff
 
 
+def _cache(torch, dec, cfg):
+    """Views of the decoder's K and V cache, [layer][kv head][position][slot]:
+    they follow the logits in its memory, each region padded to 256 bytes."""
+    from mod_amd.ops import lib
+    typ, size = ("<f4", 4) if cfg.kv_dtype == "float32" else ("<f2", 2)
+    shape = (cfg.n_layers, cfg.n_kv_heads, cfg.max_seq, cfg.head_dim)
+
+    def pad(n):
+        return (n + 255) // 256 * 256
+
+    class At:
+        def __init__(self, p):
+            self.__cuda_array_interface__ = {"shape": shape, "typestr": typ, "data": (p, False), "version": 2}
+
+    k = lib.pio_qwen3_logits(dec._h) + pad(4 * cfg.vocab)
+    return [torch.as_tensor(At(p), device="cuda:0") for p in (k, k + pad(int(np.prod(shape)) * size))]
+
+
+@pytest.mark.parametrize("kv_dtype", ["float32", "float16"])
+@pytest.mark.parametrize("P,at", [(100, 70), (300, 283), (40, 31)])
+def test_prefill_value_of_inf_stays_behind_its_position(torch_dev, kv_dtype, P, at):
+    """A token whose value row holds an inf (past the range of the cache's type)
+    leaves the positions before it as they are without it: the second layer's
+    keys and values, which carry the first one's attention. The batches keep the
+    keys of a workgroup whole (100, 40) and split them (300)."""
+    import torch
+    from mod_amd.qwen3 import Qwen3Int8Decoder, random_weights
+    cfg, _ = _small(max_seq=320, kv_dtype=kv_dtype)
+    w = random_weights(cfg, seed=65)
+    w["embed"] = w["embed"].copy()
+    L = w["layers"][0]
+    row = (cfg.n_heads + cfg.n_kv_heads) * 128 + 3        # value dim 3 of kv head 0
+    w["embed"][7] = L["w_qkv"][row]                       # aligned with token 7: about 7 times any other's
+    top = np.sqrt(cfg.hidden * float((L["w_qkv"][row].astype(np.float64) ** 2).sum()))
+    L["s_qkv"][row] = 1.5 * (3.4e38 if kv_dtype == "float32" else 65504.0) / top
+    L["b_qkv"][row] = 0
+    L["w_o"][:, [3, 131]] = 0                             # that dim of the heads that read it
+    dec = Qwen3Int8Decoder(cfg, w)
+    prompt = np.random.default_rng(66).integers(8, cfg.vocab, size=P).astype(np.int32)
+    _say(f"prefill with a value of inf: {kv_dtype} KV, {P} positions, at {at}")
+    rows = []
+    for tok in (8, 7):
+        prompt[at] = tok
+        dec.reset(prompt)
+        dec.prefill(P)
+        dec.read(0)
+        kc, vc = _cache(torch, dec, cfg)
+        assert bool(torch.isinf(vc[0, 0, at]).any()) == (tok == 7)
+        assert bool(torch.isfinite(vc[0, :, :at]).all())
+        rows.append([c[1, :, :at].float().cpu() for c in (kc, vc)])
+    for a, b in zip(*rows):
+        assert bool(torch.isfinite(b).all())
+        # one attention column in another order of sums; fp16 rows may round the other way
+        tol = 2e-5 if kv_dtype == "float32" else 2e-3
+        assert float((a - b).abs().max()) <= tol * float(a.abs().max())
+
+
 def test_prefill_refuses_generated_positions(torch_dev):
     from mod_amd.ops import RocmError
     from mod_amd.qwen3 import Qwen3Int8Decoder, random_weights
