@@ -32,7 +32,8 @@
 // of 4 sequences over 2047 keys: 578 -> 27 us (18 on the VALU kernel); causal over 1021
 // positions: 462 -> 57 us. Bound by the fp32 MFMA (35 us of it in the first)
 // and by the softmax between its two products, which two waves per SIMD only
-// partly cover. Error against 64 bits 3.1e-7 (was 5.2e-7) and 2.3e-7 (8.2e-7).
+// partly cover. Error against 64 bits 3.1e-7 (was 5.2e-7) and 1.8e-7 (8.2e-7); with
+// few keys see AT_FINE_KEYS.
 #include "attention.hpp"
 #include "wf_planes.hpp"
 
@@ -51,6 +52,14 @@ typedef _Float16 at_h8 __attribute__((ext_vector_type(8)));
 constexpr int AT_COLS = 32;    // (query, head) pairs per workgroup
 constexpr int AT_KEYS = 32;    // keys per tile
 constexpr int AT_WAVES = 4;
+// Keys up to which a column tile's scores are summed in chains of 8 terms, added as
+// a tree: with few keys their rounding is the larger part of the result's. Error
+// against 64 bits (x 1e-7) at 2 / 16 / 32 / 64 / 96 keys of 128 dims: 0.61 / 1.24 /
+// 1.52 / 1.62 / 1.68, and 0.75 / 1.50 / 1.82 / 1.94 / 2.00 in 4 chains, beside 0.62 /
+// 1.24 / 1.52 / 1.89 / 2.18 of a kernel that adds a score's 128 products as a tree,
+// which grows with the keys (5.9 at 1024; 4 chains 2.2). Costs 0.6 us (64 queries and
+// keys), and all the prompt's tiles in 8 chains would cost 2 %.
+constexpr int AT_FINE_KEYS = 96;
 constexpr int AT_VEC_COLS = 4; // columns per kv head up to which the VALU kernel serves
 
 struct AttnParams {
@@ -110,7 +119,7 @@ __device__ __forceinline__ at_f4 at_finish(const AttnArgs& a, int b, int g, int 
                                            float l) {
     constexpr bool PAIR = sizeof(KT) == 2;
     constexpr int U = 4;                   // keys at a time
-    const at_f4 r = v * (1.0f / l);
+    const at_f4 r = v / l;
     bool odd = false;
 #pragma unroll
     for (int j = 0; j < 4; j++) odd |= !(fabsf(r[j]) <= FLT_MAX);
@@ -259,6 +268,48 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams 
         else return (float)kr[c][e];
     };
 
+    // One chain of a score's terms: n groups of 8 from c.
+    auto chain = [&](int c, int n) {
+        at_v16f t;
+#pragma unroll
+        for (int e = 0; e < 16; e++) t[e] = 0.f;
+#pragma unroll
+        for (int i = c; i < c + n; i++) {
+            const at_f4 qv = *(const at_f4*)(at_lds + ((2 * i + h) * AT_COLS + col) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; e++) t = __builtin_amdgcn_mfma_f32_32x32x2f32(k_at(i, e), qv[e], t, 0, 0, 0);
+        }
+        return t;
+    };
+    const bool fine = limit_all <= AT_FINE_KEYS;
+    auto scores_fine = [&] {
+        constexpr int LV = D == 128 ? 3 : 2;
+        at_v16f level[LV], sum;
+#pragma unroll
+        for (int p2 = 0; p2 < NC / 2; p2++) {
+            sum = chain(2 * p2, 1);
+            sum += chain(2 * p2 + 1, 1);
+#pragma unroll
+            for (int i = 0; i < LV; i++) {
+                asm volatile("" : "+v"(sum));   // formed here: sunk past the branches, all chains would be held
+                if (!(p2 >> i & 1)) {
+                    level[i] = sum;
+                    break;
+                }
+                sum += level[i];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return sum;
+    };
+    // 4 chains: half the rounding of one
+    auto scores = [&] {
+        at_v16f s = chain(0, NC / 4);
+#pragma unroll
+        for (int ch = 1; ch < 4; ch++) s += chain(ch * (NC / 4), NC / 4);
+        return s;
+    };
+
     int kt = kt0 + w;
     if (kt < kt1) {
         load_k(kt, 0);
@@ -267,23 +318,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams 
     for (; kt < kt1; kt += AT_WAVES) {
         load_v(kt, 0);
         __builtin_amdgcn_sched_barrier(0);
-        // scores as 4 chains of D / 4 terms, added: half the rounding of one
-        // chain, whose error is the larger part of the probabilities'
-        at_v16f s;
-#pragma unroll
-        for (int ch = 0; ch < 4; ch++) {
-            at_v16f t;
-#pragma unroll
-            for (int e = 0; e < 16; e++) t[e] = 0.f;
-#pragma unroll
-            for (int c = ch * (NC / 4); c < (ch + 1) * (NC / 4); c++) {
-                const at_f4 qv = *(const at_f4*)(at_lds + ((2 * c + h) * AT_COLS + col) * 4);
-#pragma unroll
-                for (int e = 0; e < 4; e++) t = __builtin_amdgcn_mfma_f32_32x32x2f32(k_at(c, e), qv[e], t, 0, 0, 0);
-            }
-            if (ch == 0) s = t;
-            else s += t;
-        }
+        at_v16f s = fine ? scores_fine() : scores();
         __builtin_amdgcn_sched_barrier(0);
         load_v(kt, 1);
         __builtin_amdgcn_sched_barrier(0);
@@ -306,14 +341,18 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams 
         }
         mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
         const float corr = expf(m - mt);
-        float sum = 0.f;
+        float sum[16];                     // added as a tree
 #pragma unroll
         for (int e = 0; e < 16; e++) {
             s[e] = expf(s[e] - mt);
             if (edge && t0 + 8 * (e >> 2) + 4 * h + (e & 3) >= limit) s[e] = 0.f;
-            sum += s[e];
+            sum[e] = s[e];
         }
-        l = l * corr + sum;
+#pragma unroll
+        for (int n = 8; n >= 1; n >>= 1)
+#pragma unroll
+            for (int e = 0; e < n; e++) sum[e] += sum[e + n];
+        l = l * corr + sum[0];
         if (__any(mt != m)) {
 #pragma unroll
             for (int n = 0; n < NT; n++)
@@ -456,15 +495,17 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_vec_kernel(AttnParams p
         float s[C];
 #pragma unroll
         for (int c = 0; c < C; c++) {
-            at_f4 d = {0.f, 0.f, 0.f, 0.f};
+            at_f4 d[KL / 8];               // chains of 8 terms, added as a tree
 #pragma unroll
             for (int k = 0; k < KL; k++) {
                 const at_f4 qv = ((const at_f4*)&qs[c][8 * k])[qh];
+                at_f4& dk = d[k / 8];
 #pragma unroll
-                for (int e = 0; e < 4; e++) d[e] = fmaf(kr[k][e], qv[e], d[e]);
+                for (int e = 0; e < 4; e++) dk[e] = k % 8 ? fmaf(kr[k][e], qv[e], dk[e]) : kr[k][e] * qv[e];
                 if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // not all of q's reads at once
             }
-            s[c] = (d[0] + d[1]) + (d[2] + d[3]);
+            if (KL == 16) d[0] += d[KL / 8 - 1];
+            s[c] = (d[0][0] + d[0][1]) + (d[0][2] + d[0][3]);
             asm volatile("" : "+v"(s[c]));   // formed here: sunk past the next loads, K would be held twice
         }
         if (kt + AT_WAVES < kt1) load_k(kt + AT_WAVES);
