@@ -214,29 +214,39 @@ def _ptr(x) -> int | None:
     if x is None or type(x) is int:
         return x
     try:
-        return x.data_ptr()
+        p = x.data_ptr()
     except AttributeError:
         if isinstance(x, int):
             return x
+        if hasattr(x, "data_ptr"):   # raised inside the object's own method
+            raise
         raise TypeError(f"cannot take a device pointer of {type(x)}") from None
+    return p if type(p) is int else int(p)
 
 
 # dtype object -> element-type code, filled as dtypes are seen: forming the
-# name for each argument was 1.3 us of a 5.3 us call whose kernel takes 2.9
+# name for each argument was 1.3 us of a 5.3 us call whose kernel takes 2.9.
+# Bounded, as a caller's own class may give a new dtype object every time.
+_MISSING = object()
 _dtype_seen: dict = {}
+_DTYPE_SEEN_MAX = 64
 
 
 def _dt(x, default=F32) -> int:
     """Element-type code of a torch tensor (or the default for raw pointers)."""
-    d = getattr(x, "dtype", None)
-    if d is None:
+    d = getattr(x, "dtype", _MISSING)
+    if d is _MISSING:
         return default
-    code = _dtype_seen.get(d)
-    if code is None:
-        name = str(d).replace("torch.", "")
-        if name not in _DTYPE_CODES:
-            raise TypeError(f"unsupported dtype {d}")
-        code = _dtype_seen[d] = _DTYPE_CODES[name]
+    try:
+        return _dtype_seen[d]
+    except (KeyError, TypeError):    # TypeError: a dtype object without a hash
+        pass
+    name = str(d).replace("torch.", "")
+    if name not in _DTYPE_CODES:
+        raise TypeError(f"unsupported dtype {d}")
+    code = _DTYPE_CODES[name]
+    if len(_dtype_seen) < _DTYPE_SEEN_MAX and d.__hash__ is not None:
+        _dtype_seen[d] = code
     return code
 
 

@@ -49,6 +49,61 @@ def test_no_unexpected_dynamic_exports():
     assert not extra, f"exported but not declared: {extra}"
 
 
+def test_raw_layer_arguments():
+    """Pointers and element types of what the raw layer takes: torch tensors,
+    integers, None, and any object with a data_ptr() and a dtype of the right
+    name (a pointer as a numpy integer, a dtype without a hash or a new one on
+    every access)."""
+    import numpy as np
+    import torch
+    from mod_amd import ops
+
+    class Name:
+        def __init__(self, name):
+            self.name = name
+
+        def __str__(self):
+            return self.name
+
+        def __eq__(self, other):     # and so no hash
+            return self is other
+
+    class Fresh:
+        def __str__(self):
+            return "float16"
+
+    class Array:
+        dtype = Name("torch.int8")
+
+        def data_ptr(self):
+            return np.int64(4096)
+
+    class Broken:
+        def data_ptr(self):
+            return self.storage.pointer
+
+    t = torch.zeros(4)
+    assert ops._ptr(t) == t.data_ptr() and ops._ptr(None) is None and ops._ptr(64) == 64
+    assert type(ops._ptr(Array())) is int and ops._ptr(Array()) == 4096
+    with pytest.raises(AttributeError, match="storage"):
+        ops._ptr(Broken())
+    with pytest.raises(TypeError, match="device pointer"):
+        ops._ptr("x")
+    for name, dt in (("float32", torch.float32), ("float16", torch.float16), ("int8", torch.int8)):
+        assert ops._dt(torch.zeros(1, dtype=dt)) == ops._DTYPE_CODES[name]
+    assert ops._dt(64) == ops.F32 and ops._dt(64, ops.F16) == ops.F16
+    assert ops._dt(Array()) == ops._DTYPE_CODES["int8"]
+    a = Array()
+    for dtype in (None, torch.float64, Name("float63")):
+        a.dtype = dtype
+        with pytest.raises(TypeError, match="unsupported dtype"):
+            ops._dt(a)
+    for _ in range(1000):
+        a.dtype = Fresh()
+        assert ops._dt(a) == ops._DTYPE_CODES["float16"]
+    assert len(ops._dtype_seen) <= 64
+
+
 def test_ctensor_layout_matches_reference_struct():
     from mod_amd.ops import CTensor
     assert [f[0] for f in CTensor._fields_] == ["data", "shape", "ndim", "size", "device_id"]
