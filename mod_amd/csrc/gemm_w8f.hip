@@ -666,15 +666,16 @@ int gemm_w8_planes(const int8_t* xp, const int8_t* w, const float* s_w, const fl
                  : run_w8p<float, false>(xp, w, s_w, bias, y, ldy, M, N, K, &ws, part, splits, st);
 }
 
-// act = silu(g) * u as planes, [g|u] the linear of planes xp, where the GEMM's
-// epilogue can form it (*done); else nothing is launched.
-int gemm_w8_planes_swiglu(const int8_t* xp, const int8_t* w, const float* s_w, int8_t* act, int M, int I, int K, bool* done,
+// Whether the gate_up GEMM of M rows can form silu(g) * u in its epilogue
+// (gemm_w8_planes_swiglu).
+bool w8_planes_swiglu_fits(int M, int I) { return I % 64 == 0 && w8p_wide(M, 2 * I); }
+
+// act = silu(g) * u as planes, [g|u] the linear of planes xp.
+int gemm_w8_planes_swiglu(const int8_t* xp, const int8_t* w, const float* s_w, int8_t* act, int M, int I, int K,
                           hipStream_t st) {
     PIO_REQUIRE(xp && w && s_w && act && M > 0 && I > 0 && K > 0 && K % 16 == 0 && aligned16(xp) && aligned16(w) &&
-                    aligned16(act),
+                    aligned16(act) && w8_planes_swiglu_fits(M, I),
                 "gemm_w8_planes_swiglu: bad operands");
-    *done = I % 64 == 0 && w8p_wide(M, 2 * I);
-    if (!*done) return PIO_OK;
     W8pParams p{};
     p.xp = xp; p.w = w; p.s_w = s_w; p.y = act;
     p.M = M; p.N = 2 * I; p.K = p.ks = K;

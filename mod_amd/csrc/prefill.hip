@@ -23,6 +23,7 @@
 #include "decode.hpp"
 #include "wf_planes.hpp"
 
+#include <algorithm>
 #include <float.h>
 #include <math.h>
 
@@ -30,7 +31,8 @@ namespace pio {
 
 int gemm_w8_planes(const int8_t* xp, const int8_t* w, const float* s_w, const float* bias, float* y, int64_t ldy, int M,
                    int N, int K, bool resid, Scratch& ws, const float** part, int* splits, hipStream_t st);
-int gemm_w8_planes_swiglu(const int8_t* xp, const int8_t* w, const float* s_w, int8_t* act, int M, int I, int K, bool* done,
+bool w8_planes_swiglu_fits(int M, int I);
+int gemm_w8_planes_swiglu(const int8_t* xp, const int8_t* w, const float* s_w, int8_t* act, int M, int I, int K,
                           hipStream_t st);
 
 // x[m] = embed[ids[pos0 + m]] (an out-of-range id reads row 0, as the step).
@@ -239,20 +241,25 @@ int prefill(Qwen3Dec* d, int M, bool logits) {
     PIO_REQUIRE(H % 16 == 0 && I % 16 == 0, "pio_qwen3_prefill: hidden and intermediate must be multiples of 16");
     hipStream_t st = d->st;
     // activations of the batch: x, qkv and [g|u] in fp32; the linears' inputs (h,
-    // the normed x; the attention's output; act) as planes
+    // the normed x; o, the attention's output; act) as planes. [g|u], where the
+    // gate_up GEMM does not form act itself, lies over qkv and o, which are done
+    // with by then: planes take 6 bytes a value, and so the batch takes no more
+    // than in fp32.
     auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t b_x = al((size_t)M * H * 4), b_qkv = al((size_t)M * nqkv * 4), b_gu = al((size_t)M * 2 * I * 4);
+    const bool fused = w8_planes_swiglu_fits(M, I);
+    const size_t b_x = al((size_t)M * H * 4), b_qkv = al((size_t)M * nqkv * 4);
+    const size_t b_gu = fused ? 0 : al((size_t)M * 2 * I * 4);
     const size_t b_h = al(wf_planes_bytes(M, H)), b_o = al(wf_planes_bytes(M, nq * D)), b_act = al(wf_planes_bytes(M, I));
     Scratch ws;
-    PIO_TRY(ws.get(b_x + b_qkv + b_gu + b_h + b_o + b_act, st));
+    PIO_TRY(ws.get(b_x + b_h + b_act + std::max(b_qkv + b_o, b_gu), st));
     char* at_ = (char*)ws.ptr;
     auto take = [&](size_t b) { char* r = at_; at_ += b; return r; };
     float* x = (float*)take(b_x);
-    float* qkv = (float*)take(b_qkv);
-    float* gu = (float*)take(b_gu);
     int8_t* h = (int8_t*)take(b_h);
-    int8_t* o = (int8_t*)take(b_o);
     int8_t* act = (int8_t*)take(b_act);
+    float* gu = (float*)at_;
+    float* qkv = (float*)take(b_qkv);
+    int8_t* o = (int8_t*)take(b_o);
     const int rb = wf_row_blocks(M);
     pf_embed_kernel<<<M, 256, 0, st>>>(d->embed, d->ids, pos0, x, H, c.vocab);
     PIO_LAUNCHED();
@@ -322,19 +329,16 @@ int prefill(Qwen3Dec* d, int M, bool logits) {
                 pf_rmsnorm_kernel<<<rb, 256, 0, st>>>(x, L.post_norm, h, M, H, c.rms_eps);
             PIO_LAUNCHED();
         }
-        {
-            bool fused;
-            PIO_TRY(gemm_w8_planes_swiglu(h, L.w_gu, L.s_gu, act, M, I, H, &fused, st));
-            if (!fused) {
-                Scratch pw;
-                const float* part;
-                int sp;
-                PIO_TRY(gemm_w8_planes(h, L.w_gu, L.s_gu, nullptr, gu, 2 * I, M, 2 * I, H, false, pw, &part, &sp,
-                                       st));
-                pf_swiglu_kernel<<<dim3(ceil_div(I, 1024), rb), 256, 0, st>>>(gu, sp ? part : nullptr, sp, M, I,
-                                                                                  L.s_gu, act);
-                PIO_LAUNCHED();
-            }
+        if (fused) {
+            PIO_TRY(gemm_w8_planes_swiglu(h, L.w_gu, L.s_gu, act, M, I, H, st));
+        } else {
+            Scratch pw;
+            const float* part;
+            int sp;
+            PIO_TRY(gemm_w8_planes(h, L.w_gu, L.s_gu, nullptr, gu, 2 * I, M, 2 * I, H, false, pw, &part, &sp, st));
+            pf_swiglu_kernel<<<dim3(ceil_div(I, 1024), rb), 256, 0, st>>>(gu, sp ? part : nullptr, sp, M, I, L.s_gu,
+                                                                              act);
+            PIO_LAUNCHED();
         }
         {
             Scratch pw;

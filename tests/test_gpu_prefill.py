@@ -172,6 +172,28 @@ def test_prefill_refuses_generated_positions(torch_dev):
         dec.prefill(1)
 
 
+@pytest.mark.parametrize("intermediate", [3072, 3088])
+def test_prefill_memory(torch_dev, intermediate):
+    """What a batch of 2048 positions takes from the allocator is no more than its
+    activations in fp32 (x, its norm, qkv, the attention's output, [g|u], act),
+    with the SwiGLU in the gate_up GEMM (3072) and as a kernel of its own. At this
+    size no linear and no attention splits a sum, so nothing else is taken."""
+    from mod_amd import ops
+    from mod_amd.qwen3 import Qwen3Int8Decoder, random_weights
+    cfg, _ = _small(max_seq=2048, intermediate=intermediate)
+    dec = Qwen3Int8Decoder(cfg, random_weights(cfg, seed=67))
+    prompt = np.random.default_rng(68).integers(0, cfg.vocab, size=2048).astype(np.int32)
+    dec.reset(prompt)
+    before = ops.pool_stats()["reserved"]
+    dec.prefill(2048)
+    dec.read(0)
+    taken = ops.pool_stats()["reserved"] - before
+    heads, kv = cfg.n_heads * cfg.head_dim, cfg.n_kv_heads * cfg.head_dim
+    row = 4 * (2 * cfg.hidden + (heads + 2 * kv) + heads + 3 * intermediate)
+    _say(f"2048 positions, I={intermediate}: {taken} bytes taken, {2048 * row} in fp32")
+    assert 0 < taken <= 2048 * row
+
+
 @pytest.mark.parametrize("mode", ["persistent", "graph"])
 def test_prefill_then_decode_small(torch_dev, mode):
     """Prompt in one batch, then greedy steps: the steps' logits (the first
