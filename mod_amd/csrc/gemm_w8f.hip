@@ -628,8 +628,14 @@ static int run_w8p_tiles(W8pParams p, int blocks, int min_steps, Scratch* ws, co
 }
 
 // Whether the planes GEMM takes these sizes in 128 x 128 tiles (see run_w8p; such a
-// plan never splits K).
-static bool w8p_wide(int M, int N) { return N >= 6144 && (int64_t)ceil_div(M, 128) * ceil_div(N, 128) >= 160; }
+// plan never splits K). Up to 64 rows the narrower tiles are as fast or faster at
+// any width, as half the wide tile's waves would repeat rows: (M, N, K) = (13,
+// 24576, 4096) 73 us wide and 47 in 32 x 128 tiles, (32, 151936, 1024) 105 / 60, (33,
+// 24576, 4096) 74 / 75, (64, 151936, 1024) 106 / 96 in 64 x 64; from 65 rows on the
+// wide ones: (65, 24576, 4096) 75 / 103, (100, 20480, 1024) 25 / 28.
+static bool w8p_wide(int M, int N) {
+    return M > 64 && N >= 6144 && (int64_t)ceil_div(M, 128) * ceil_div(N, 128) >= 160;
+}
 
 template <typename YT, bool RESID>
 static int run_w8p(const int8_t* xp, const int8_t* w, const float* s_w, const float* bias, YT* y, int64_t ldy, int M,

@@ -825,6 +825,8 @@ def test_skinny_paths_full_size_properties(env):
     (33, 9001, 2064),     # 64 x 64 tiles, K slices
     (129, 5003, 1040),    # 128 x 64: one row and 11 columns in the last tiles
     (420, 6200, 1040),    # 128 x 128
+    (32, 20500, 1040), (64, 20500, 1040),   # wide outputs of few rows: 32 x 128 and 64 x 64
+    (65, 20500, 1040),    # 128 x 128 with 65 rows
     (1000, 1000, 12304),  # two chunks of rows; one slice of K longer than the rest
 ])
 def test_w8_linear_planes(env, M, N, K):
