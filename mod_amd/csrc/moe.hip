@@ -2,7 +2,9 @@
 // (Qwen3Coder30BMoE.forward, ip/models/qwen3_coder_30b/model.py:308-353: a
 // D2H sync per slot, one gather/MLP/scatter call chain per expert, an atomic
 // and therefore order-dependent scatter-add) with six launches and a
-// deterministic combine:
+// deterministic combine (up to 8 tokens one launch routes, quantizes and groups,
+// and one or two tokens take GEMMs of their own, which requantize: "few tokens"
+// below):
 //
 //  1. route:   p = softmax(logits) exactly as tensor_softmax (tensor_ops.c:351-368:
 //              max seeded with -1e9, exp(x - max), multiply by 1/sum); top-k by
@@ -411,7 +413,7 @@ static void launch_grouped(const GroupedParams& g, dim3 grid, int nk, hipStream_
     }
 }
 
-// -------------------------------------------------------- one or two tokens ---
+// --------------------------------------------------------------- few tokens ---
 // A decode step: the six launches above move the 8 experts' 38 MB in 14 us and
 // take 36, most of it launches, and blocks for every expert without a token.
 // Here one block routes, quantizes and groups the tokens (and lists the experts
@@ -421,18 +423,18 @@ static void launch_grouped(const GroupedParams& g, dim3 grid, int nk, hipStream_
 // v_mfma_i32_16x16x64_i8, two sets of MS_SET K values in flight, with the
 // activation rows in LDS; the down kernel quantizes its h rows itself. Same
 // integer sums, scales and order as above, so the same bits.
-// Qwen3-30B-A3B layer: T = 1 36.4 -> 25.2 us. From T = 3 the path above is the
-// faster one (41 / 46 us at 3, 86 / 114 at 16): these loads cover half a line of
+// Qwen3-30B-A3B layer: T = 1 36.4 -> 25.2 us. From T = 3 the GEMMs above are the
+// faster ones (41 / 46 us at 3, 86 / 114 at 16): these loads cover half a line of
 // a row each and stream at 4 TB/s, its tiles at 4.6 and up.
 constexpr int MS_MAX_T = 2;        // tokens (and rows of an expert)
 // Tokens up to which the front kernel replaces the route and group launches:
 // one round of its 16 waves, a wave per job. Above MS_MAX_T the GEMMs are the
-// general ones, on blocks for the listed experts only: T = 4 / 5 / 8 of the same
-// layer 47.7 / 52.6 / 65.3 -> 45.1 / 49.6 / 63.0 us. T = 3 was slower in each of two
-// runs (41.4 -> 42.7 us, cause not found) and keeps the general path.
+// general ones, on blocks for the listed experts only: T = 3 / 4 / 5 / 8 of the same
+// layer 42.3 / 47.7 / 52.6 / 65.3 -> 43.1 / 45.1 / 49.6 / 63.0 us, of a layer of 64
+// experts (4 per token, H 1024, I 512) 28.4 -> 23.7 at 3. The one loss, 2 %, is in
+// gate_up (19.6 -> 20.8): 288 blocks, all started at once, are one and a bit per CU.
 constexpr int FR_MAX_T = 8;
 constexpr int FR_MAX_P = 64 * FR_MAX_T;   // (token, slot) pairs
-static bool front_path(int T) { return T <= MS_MAX_T || (T > 3 && T <= FR_MAX_T); }
 constexpr int MS_SET = 512;        // K values of a wave's rows per register set
 constexpr int MS_LOADS = MS_SET / 64;
 
@@ -798,7 +800,7 @@ int moe_w8a8(const void* x, int x_dtype, const float* logits, const int8_t* w_gu
         PIO_LAUNCHED();
         return PIO_OK;
     };
-    const bool front = front_path(T);
+    const bool front = T <= FR_MAX_T;
     if (front) {
         MoeFront f{logits, x, H, T, E, top_k, renorm, w.topk_w, w.topk_id, w.qx, w.sx, w.amax, w.offsets, w.row_token,
                    w.pos_of_pair, w.active};

@@ -943,7 +943,7 @@ def test_moe_logits_without_an_order(env, T):
     (1152, 1152, 9, 9, "float32"),                 # every expert takes every token
     (256, 256, 1024, 64, "float16")])              # the most experts and slots
 def test_moe_few_tokens_equal_general_path(env, H, I, E, k, xdt):
-    """4 to 8 tokens are routed and grouped by one block, and only the experts
+    """3 to 8 tokens are routed and grouped by one block, and only the experts
     it lists get GEMM blocks: each call must equal, bit for bit, its rows of a
     12-token call, which the general path takes."""
     torch, ops, d = env
