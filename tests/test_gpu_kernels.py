@@ -873,13 +873,13 @@ def test_w8_linear_planes(env, M, N, K):
     (4096, 256, 1024, 64, "float16", False)])      # the most experts, slots and columns
 def test_moe_one_or_two_tokens_equal_general_path(env, H, I, E, k, xdt, renorm):
     """One or two tokens take kernels of their own; a token's output does not
-    depend on the others, so each must equal, bit for bit, its row of a 6-token
+    depend on the others, so each must equal, bit for bit, its row of a 12-token
     call, which takes the general path (and whose results the oracle tests
     hold)."""
     torch, ops, d = env
     _say(f"moe one or two tokens H={H} I={I} E={E} k={k}")
     g = torch.Generator(device=d).manual_seed(H + E)
-    T = 6
+    T = 12
     x = torch.randn((T, H), generator=g, device=d).to(getattr(torch, xdt))
     x[3] = 0                                        # zero rows quantize with scale 1
     logits = torch.randn((T, E), generator=g, device=d)
@@ -900,10 +900,12 @@ def test_moe_one_or_two_tokens_equal_general_path(env, H, I, E, k, xdt, renorm):
             assert torch.equal(out, full[t:t + n]), (t, n, odt)
 
 
-@pytest.mark.parametrize("T", [1, 2, 6])
+@pytest.mark.parametrize("T", [1, 2, 3, 6, 9, 40])
 def test_moe_logits_without_an_order(env, T):
     """Logits with a NaN or an inf, or only -inf, give NaN probabilities: the
-    token gets valid, distinct experts and a NaN output, the others their own."""
+    token gets valid, distinct experts and a NaN output, the others their own.
+    1 and 2 tokens take kernels of their own, 3 to 8 the one-block front, more
+    the general route and grouping."""
     torch, ops, d = env
     H, I, E, k = 128, 128, 9, 3
     g = torch.Generator(device=d).manual_seed(T)
