@@ -159,6 +159,31 @@ def test_prefill_value_of_inf_stays_behind_its_position(torch_dev, kv_dtype, P, 
         assert float((a - b).abs().max()) <= tol * float(a.abs().max())
 
 
+def test_prefill_fp16_keys_split(torch_dev):
+    """fp16 KV where the attention splits its keys over workgroups: a batch of
+    300 positions, then a late one of 40, against the oracle and against batches
+    of at most 100, the first two of which keep them whole (the bar of the first
+    test: fp16 cache rows that round the other way)."""
+    from mod_amd.qwen3 import Qwen3Int8Decoder, random_weights
+    cfg, rcfg = _small(max_seq=384, kv_dtype="float16")
+    w = random_weights(cfg, seed=69)
+    dec = Qwen3Int8Decoder(cfg, w)
+    prompt = np.random.default_rng(70).integers(0, cfg.vocab, size=340).astype(np.int32)
+    logits = []
+    for sizes in ((300, 40), (100, 100, 100, 40)):
+        _say(f"fp16 KV, batches of {sizes}")
+        dec.reset(prompt)
+        for n in sizes[:-1]:
+            dec.prefill(n)
+        dec.prefill(sizes[-1], logits=True)
+        logits.append(dec.read(0, with_logits=True)[1].copy())
+        _against_oracle(logits[-1][None], prompt, [339], rcfg, w, f"fp16 KV, batches of {sizes}")
+    rms = float(np.sqrt(np.mean(logits[0].astype(np.float64) ** 2)))
+    diff = float(np.abs(logits[0] - logits[1]).max()) / rms
+    _say(f"max diff {diff:.2e} x rms")
+    assert diff <= 2e-3, diff
+
+
 def test_prefill_refuses_generated_positions(torch_dev):
     from mod_amd.ops import RocmError
     from mod_amd.qwen3 import Qwen3Int8Decoder, random_weights
