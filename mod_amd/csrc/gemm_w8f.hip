@@ -603,12 +603,14 @@ static int run_w8p_tiles(W8pParams p, int blocks, int min_steps, Scratch* ws, co
     const int tiles = p.m_tiles * p.n_tiles;
     p.per_xcd = ceil_div(tiles, 8);
     const int steps = ceil_div(p.K, 64);
-    // Few rows, many tiles: as many slices as fill the blocks, not a power of two
-    // (96 tiles: 5 slices, 480 blocks, against 4 that give half the CUs two blocks
-    // and half one: (13, 12288, 4096) 24.7 -> 22.6 us, (32, 12288, 2064) 21.4 -> 20.3).
-    // At 64 tiles and fewer the powers of two fill them as well with fewer
-    // partials ((32, 5003, 4096), 40 tiles: 18.55 us against 18.65).
-    int splits = WM > 1 || tiles <= 64 ? wf_splits(tiles, p.K, 64, blocks, min_steps)
+    // Few rows, more than 32 tiles: as many slices as fill the blocks, not a power
+    // of two (96 tiles: 5 slices, 480 blocks, against 4 that give half the CUs two
+    // blocks and half one: (13, 12288, 4096) 24.7 -> 22.6 us; 56 tiles: (32, 7168, 8192)
+    // 27.7 -> 25.9; 48: (32, 6144, 4096) 18.4 -> 18.1; 40: 18.5 -> 18.4). Fewer tiles
+    // have so many slices that the powers of two fill the CUs too, and each further
+    // slice is another M x N of partials: (32, 2305, 12288), 19 tiles, 16 slices 24.2
+    // us, 26 slices 26.0; 24 tiles 22.3 / 22.5.
+    int splits = WM > 1 || tiles <= 32 ? wf_splits(tiles, p.K, 64, blocks, min_steps)
                                        : std::max(1, std::min(blocks / tiles, steps / min_steps));
     p.ks = ceil_div(steps, splits) * 64;
     splits = ceil_div(p.K, p.ks);

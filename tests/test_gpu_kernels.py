@@ -822,6 +822,7 @@ def test_skinny_paths_full_size_properties(env):
 
 @pytest.mark.parametrize("M,N,K", [
     (9, 16400, 4112),     # 32 x 128 tiles; a last K step of 16
+    (37, 4096, 4112), (20, 4200, 8208),     # 64 x 64; 33 tiles of 32 x 128 in 15 slices
     (33, 9001, 2064),     # 64 x 64 tiles, K slices
     (129, 5003, 1040),    # 128 x 64: one row and 11 columns in the last tiles
     (420, 6200, 1040),    # 128 x 128
