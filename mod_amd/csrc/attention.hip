@@ -640,12 +640,12 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
 }
 
 bool attn_mfma_supported(const AttnArgs& a) {
-    // causal: the decoder's cache (head_dim 128); fp16 keys only there
+    // causal: the decoder's prompt (head_dim 128, planes out); fp16 keys only there
     if (a.D != 128 && !(a.D == 64 && !a.causal)) return false;
     if (a.kv16 && !a.causal) return false;
     if (a.H % a.Hk || a.kv_t >= 1 << 25 || a.q_s % 4 || a.o_s % 4 || a.q_b % 4 || a.o_b % 4 || a.kv_t % 8 || a.kv_h % 8 || a.kv_b % 8)
         return false;
-    return aligned16(a.q) && aligned16(a.k) && aligned16(a.v) && aligned16(a.out);
+    return aligned16(a.q) && aligned16(a.k) && aligned16(a.v) && aligned16(a.out) && aligned16(a.planes);
 }
 
 template <int D, bool PAIR, bool CAUSAL>
@@ -681,6 +681,9 @@ static int attn_vec_launch(const AttnParams& p, hipStream_t st) {
 }
 
 int attn_mfma(const AttnArgs& a, hipStream_t st) {
+    PIO_REQUIRE(a.B > 0 && a.S > 0 && a.T > 0 && a.Hk > 0 && (a.causal ? a.planes != nullptr : a.out != nullptr) &&
+                    attn_mfma_supported(a),
+                "attn_mfma: bad operands");
     AttnParams p{};
     p.a = a;
     p.G = a.H / a.Hk;

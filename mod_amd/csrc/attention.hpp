@@ -24,7 +24,8 @@ struct AttnArgs {
     float m_seed;         // the running maximum starts here
 };
 
-// Whether attn_mfma takes these shapes and addresses (else: the caller's own kernel).
+// Whether attn_mfma takes these shapes and addresses (else: the caller's own
+// kernel, or attn_mfma's error).
 bool attn_mfma_supported(const AttnArgs& a);
 int attn_mfma(const AttnArgs& a, hipStream_t st);
 

@@ -46,7 +46,7 @@ typedef __attribute__((address_space(1))) const wf_f4 wf_gf4;
 constexpr int WF_BK = 64;
 constexpr int WF_ROW = WF_BK * 2;   // LDS bytes per tile row of a step
 
-enum { WF_STORE = 0, WF_RESID = 1, WF_PARTIAL = 2, WF_SWIGLU = 3 };
+enum { WF_STORE = 0, WF_RESID = 1, WF_PARTIAL = 2, WF_SWIGLU = 3 };   // RESID, SWIGLU: planes kernel
 
 struct W8fParams {
     const void* x;
@@ -109,6 +109,7 @@ template <> struct WfXRegs<_Float16> { wf_v4i v[2]; };  // 16 fp16
 template <int NL, typename XT, typename YT, int EPI, int TM, int TN>
 __global__ __launch_bounds__(256) void gemm_w8f_kernel(W8fParams p) {
     static_assert((NL == 3) == std::is_same<XT, float>::value, "three bf16 parts for fp32 x, one for fp16");
+    static_assert(EPI == WF_STORE || EPI == WF_PARTIAL, "a residual is added by the planes kernel only");
     extern __shared__ __attribute__((aligned(16))) int8_t wf_lds[];
     constexpr int BM = 64 * TM, BN = 64 * TN;
     constexpr int XB = BM * WF_ROW;                    // one part's x tile
