@@ -611,8 +611,11 @@ static int run_w8p_tiles(W8pParams p, int blocks, int min_steps, Scratch* ws, co
     // have so many slices that the powers of two fill the CUs too, and each further
     // slice is another M x N of partials: (32, 2305, 12288), 19 tiles, 16 slices 24.2
     // us, 26 slices 26.0; 24 tiles 22.3 / 22.5.
-    int splits = WM > 1 || tiles <= 32 ? wf_splits(tiles, p.K, 64, blocks, min_steps)
-                                       : std::max(1, std::min(blocks / tiles, steps / min_steps));
+    // Nor in 128 x 64 tiles whose slices a reduce launch adds: (200, 2560, 3072), 80
+    // tiles, 2 slices 28.5 us, 3 slices 25.0.
+    const bool fill = (WM == 1 && tiles > 32) || (WM == 4 && !part);
+    int splits = fill ? std::max(1, std::min(blocks / tiles, steps / min_steps))
+                      : wf_splits(tiles, p.K, 64, blocks, min_steps);
     p.ks = ceil_div(steps, splits) * 64;
     splits = ceil_div(p.K, p.ks);
     if (splits == 1) return launch_w8p<YT, RESID ? WF_RESID : WF_STORE, WM, TN>(p, 1, st);
@@ -656,6 +659,18 @@ static int run_w8p(const int8_t* xp, const int8_t* w, const float* s_w, const fl
     // 1910 / 2438 / 3640.
     if (w8p_wide(M, N))
         return run_w8p_tiles<YT, RESID, 4, 4>(p, 256, 4, ws, part, splits, st);
+    // A linear by itself (no part: its K slices cost a reduce launch) of 129 to 384
+    // rows: 64 x 64 tiles where they take fewer rounds of the CUs than 128 x 64 ones,
+    // a round of them counted as 0.7 of theirs ((300, 6144, 4096), 480 tiles against
+    // 288: 65 us against 81; (160, 5003, 2064), 237 against 158: 25 / 32; not at (384,
+    // 6144, 4096), 576 against 288: 95 / 86); K slices for one block per CU, two when
+    // K is long ((230, 6144, 1024): 19 us, 27 with two; (160, 4096, 12288): 81, 79).
+    if (!part && M > 128 && M <= 384) {
+        const int tall = ceil_div(M, 128) * ceil_div(N, 64), small = ceil_div(M, 64) * ceil_div(N, 64);
+        if (tall > 128 && 14 * ceil_div(small, 256) < 20 * ceil_div(tall, 256))
+            return run_w8p_tiles<YT, RESID, 2, 1>(p, 256, 4, ws, part, splits, st);
+        return run_w8p_tiles<YT, RESID, 4, 2>(p, K > 4096 && M <= 256 ? 512 : 256, 4, ws, part, splits, st);
+    }
     if (M > 128) return run_w8p_tiles<YT, RESID, 4, 2>(p, M <= 256 ? 512 : 256, 4, ws, part, splits, st);
     if (M > 32) return run_w8p_tiles<YT, RESID, 2, 1>(p, 512, 4, ws, part, splits, st);
     return run_w8p_tiles<YT, RESID, 1, 1>(p, 512, 2, ws, part, splits, st);
@@ -706,9 +721,12 @@ static int run_w8f(const XT* x, const int8_t* w, const float* s_w, const float* 
         // 14.6, (127, 6144, 1024) 17.2 / 19.3, (509, 6144, 1024) 27 / 36, (1021,
         // 1024, 2048) 30 / 29, (1021, 1024, 3072) 37 / 41, (2048, 3072, 1024) 52 / 71,
         // (2048, 12288, 4096) 488 / 762; (40, 12288, 4096) 30 / 48, (64, 3072, 1024)
-        // 12.9 / 11.1
+        // 12.9 / 11.1. Not for 129 to 256 rows of a small weight, which would need K
+        // slices: (192, 4096, 1024) 19.9 / 19.0, (256, 2048, 2048) 19.9 / 16.4, but (192,
+        // 3072, 2048) 24.6 / 26.9.
         const double mnk = (double)M * N * K;
-        if (mnk >= (N >= 2048 ? 0.6e9 : 3e9)) {
+        const bool sliced = M > 128 && M <= 256 && N <= 4096 && (int64_t)N * K <= 5000000;
+        if (mnk >= (N >= 2048 && !sliced ? 0.6e9 : 3e9)) {
             // row chunks keep the planes within 64 MB
             const int rows = (int)std::max<int64_t>(128, ((64ll << 20) / (6ll * K)) & ~127ll);
             for (int m0 = 0; m0 < M; m0 += rows) {

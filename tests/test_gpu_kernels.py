@@ -824,7 +824,11 @@ def test_skinny_paths_full_size_properties(env):
     (9, 16400, 4112),     # 32 x 128 tiles; a last K step of 16
     (37, 4096, 4112), (20, 4200, 8208),     # 64 x 64; 33 tiles of 32 x 128 in 15 slices
     (33, 9001, 2064),     # 64 x 64 tiles, K slices
-    (129, 5003, 1040),    # 128 x 64: one row and 11 columns in the last tiles
+    (129, 5003, 1040),    # 64 x 64 where 128 x 64 would be 158 tiles: one row and 11 columns in the last ones
+    (300, 6150, 1040),    # 64 x 64 again, 485 tiles against 291
+    (200, 2500, 3088),    # 128 x 64 in 3 slices of K, the last one shorter
+    (200, 5600, 1040),    # 128 x 64, whole sums
+    (256, 4096, 1040),    # split in the GEMM: small weight
     (420, 6200, 1040),    # 128 x 128
     (32, 20500, 1040), (64, 20500, 1040),   # wide outputs of few rows: 32 x 128 and 64 x 64
     (65, 20500, 1040),    # 128 x 128 with 65 rows
