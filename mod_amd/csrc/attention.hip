@@ -281,14 +281,15 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams 
         }
         return t;
     };
+    // (causal: of 16 terms, as its 8 partial sums of a score were before)
     const bool fine = limit_all <= AT_FINE_KEYS;
     auto scores_fine = [&] {
-        constexpr int LV = D == 128 ? 3 : 2;
+        constexpr int CG = CAUSAL ? 2 : 1, PAIRS = NC / CG / 2, LV = PAIRS == 8 ? 3 : 2;
         at_v16f level[LV], sum;
 #pragma unroll
-        for (int p2 = 0; p2 < NC / 2; p2++) {
-            sum = chain(2 * p2, 1);
-            sum += chain(2 * p2 + 1, 1);
+        for (int p2 = 0; p2 < PAIRS; p2++) {
+            sum = chain(2 * p2 * CG, CG);
+            sum += chain((2 * p2 + 1) * CG, CG);
 #pragma unroll
             for (int i = 0; i < LV; i++) {
                 asm volatile("" : "+v"(sum));   // formed here: sunk past the branches, all chains would be held

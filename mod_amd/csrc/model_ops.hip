@@ -10,6 +10,7 @@
 // (PIO_OK or a negative code with the message in tensor_last_error).
 #include "attention.hpp"
 
+#include <algorithm>
 #include <climits>
 
 namespace pio {
@@ -220,9 +221,9 @@ __global__ __launch_bounds__(MO_THREADS) void mo_embed_kernel(const float* __res
 }
 
 // ---------------------------------------------------------- attention ------
-// The general kernel: head sizes and addresses that attention.hip's
-// matrix-core kernel does not take (it wants head_dim 64 or 128 and 16-byte
-// aligned rows).
+// The general kernel: head sizes and addresses that attention.hip's kernels do
+// not take (they want head_dim 64 or 128 and 16-byte aligned rows), and few keys
+// (sdpa_few_keys).
 // One block per (batch, query position, head): q [B, S, H, D], k / v
 // [B, T, Hk, D], out [B, S, H, D]. Scores q.k * scale over all T keys (no
 // mask, as the reference), softmax with max from -1e9 and the weights
@@ -454,6 +455,20 @@ PIO_EXPORT void tensor_embed(Tensor* weight, Tensor* indices, Tensor* out) {
 
 constexpr int MO_SDPA_MAX_T = 32768;   // keys held in LDS (128 KB of scores)
 
+// Whether few rows over few keys stay with the general kernel. Its blocks, one per
+// row, all run at once and walk the keys: 3.2 us and 0.13 per key (128 dims; 0.10
+// with 64). attention.hip's kernels take a tile of 32 keys for one key's price, a
+// wave's serial work: 5 / 7 us of VALU work for 2 / 4 columns per kv head, 10 to 12
+// on the MFMAs (7 to 8 with 64 dims). B x S x H rows over T keys, 128 dims: 1 x 5 x 16
+// over 5 4.2 us here and 10.5 there, 1 x 48 x 16 over 48 10.0 / 11.8, 1 x 64 x 16 over
+// 64 13.2 / 11.8, 1 x 1 x 16 over 16 5.2 / 5.1, over 32 7.4 / 5.1, 1 x 1 x 32 over 24
+// 6.3 / 7.3; 64 dims: 1 x 20 x 16 over 36 7.2 / 7.6, 1 x 48 x 16 over 48 8.8 / 7.7;
+// more rows run in rounds: 2 x 33 x 32 over 33 15.0 / 11.9.
+static bool sdpa_few_keys(int B, int S, int T, int H, int Hk, int D) {
+    const int cols = S * (H / Hk);
+    return (int64_t)B * S * H <= 12 * D && T <= (D == 128 ? 8 * std::min(cols, 6) : 5 * std::min(cols, 8));
+}
+
 PIO_EXPORT int tensor_scaled_dot_product_attention_status(Tensor* q, Tensor* k, Tensor* v, Tensor* out,
                                                           float scale) {
     const char* nm = "tensor_scaled_dot_product_attention";
@@ -480,7 +495,7 @@ PIO_EXPORT int tensor_scaled_dot_product_attention_status(Tensor* q, Tensor* k, 
     at.B = B; at.S = S; at.T = T; at.H = H; at.Hk = Hk; at.D = D;
     at.scale = scale;
     at.m_seed = -1e9f;
-    if (attn_mfma_supported(at)) return attn_mfma(at, current_stream());
+    if (attn_mfma_supported(at) && !sdpa_few_keys(B, S, T, H, Hk, D)) return attn_mfma(at, current_stream());
     const size_t lds = (size_t)T * sizeof(float);
     PIO_TRY(allow_lds<mo_sdpa_kernel>(lds));
     mo_sdpa_kernel<<<(unsigned)blocks, MO_THREADS, lds, current_stream()>>>(q->data, k->data, v->data, out->data, S, T,

@@ -149,7 +149,10 @@ def _general_attention(B, q, k, v):
     (1, 11, 3, 1, 31, 128),      # 33 columns: the second tile holds one; a partial key tile
     (1, 65, 4, 4, 65, 64), (3, 1, 16, 8, 1023, 128),   # keys split over workgroups, ragged last split
     (1, 300, 8, 2, 517, 128), (2, 1, 32, 4, 4100, 64),
-    (2, 1, 8, 8, 70, 128), (1, 3, 2, 2, 33, 64), (1, 2, 4, 2, 2049, 128)])   # 1, 3 and 4 columns: the VALU kernel
+    (2, 1, 8, 8, 70, 128), (1, 3, 2, 2, 33, 64), (1, 2, 4, 2, 2049, 128),   # 1, 3 and 4 columns: the VALU kernel
+    (800, 1, 2, 1, 1, 128), (7, 16, 16, 8, 33, 128), (50, 11, 3, 1, 31, 128),   # more rows than the general kernel keeps
+    (24, 4, 16, 8, 48, 128), (25, 4, 16, 8, 48, 128), (1, 12, 4, 2, 49, 128), (3, 16, 16, 16, 40, 64),   # either side of
+    (4, 16, 16, 16, 40, 64), (1, 16, 4, 4, 41, 64), (1, 1, 8, 4, 16, 128), (1, 1, 8, 4, 17, 128)])       # that rule
 def test_attention_tiles(B, Bn, S, H, Hk, T, D):
     """The matrix-core attention at the edges of its column and key tiles and of
     its key splits, against the oracle and against the general kernel (which
@@ -216,7 +219,7 @@ def test_attention_value_range(B, Bn, S, H, Hk, T, D):
     assert np.array_equal(tq.numpy(), got, equal_nan=True)
 
 
-@pytest.mark.parametrize("Bn,S,H,Hk,D", [(2, 64, 16, 8, 128), (2, 64, 16, 16, 64), (32, 1, 32, 8, 128), (32, 2, 16, 16, 64)])
+@pytest.mark.parametrize("Bn,S,H,Hk,D", [(2, 64, 16, 8, 128), (2, 64, 16, 16, 64), (64, 1, 32, 8, 128), (32, 2, 16, 16, 64)])
 def test_attention_few_keys_error(B, Bn, S, H, Hk, D):
     """With few keys the rounding of the scores is most of the error: it is no
     larger than the general kernel's, whose scores are sums of two-term chains
