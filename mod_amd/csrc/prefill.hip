@@ -229,6 +229,142 @@ __global__ void pf_handoff_kernel(const float* __restrict__ xb, int m, int H, fl
 
 constexpr int ATT_MAX_G_PF = 4;   // query heads per KV head
 
+// Keys up to which a batch's attention runs on pf_attn_kernel: 4.7 us a layer (16
+// positions of the 0.6B shape) and 1.1 more for every 32 keys, where a wave of
+// attention.hip's kernel takes a tile of 32 keys in 13. 0.6B prompt of 16 / 64 / 96 /
+// 112 positions: 1196 / 1490 / 1778 / 1867 us on this one, 1425 / 1609 / 1838 / 1819
+// on the other; 40 positions after 100 others 1706 / 1750, 64 after 100 1808 / 1769, one
+// after 900 3501 / 1557.
+constexpr int PF_FEW_KEYS = 96;
+
+// Causal GQA attention of a short batch: row m (position p = pos0 + m), the G query
+// heads of KV head g, cache positions 0 .. p, with an online softmax over passes
+// of 32 positions, into row m of the output's planes. Per pass: 8 threads per
+// position score it (16 dims each); the first G half-waves fold the pass's scores
+// into each head's running max and sum (the scores become exp(s - max) in place);
+// then every thread folds the pass into two output dims (d and d + 64) of one or
+// two heads, over half the pass's positions. Block (m, g), 256 threads.
+template <typename KT>
+__global__ __launch_bounds__(256) void pf_attn_kernel(const float* __restrict__ qkv, int ldq, int pos0, int nq,
+                                                      int nkv, const KT* __restrict__ kc, const KT* __restrict__ vc,
+                                                      int max_seq, float scale, int8_t* __restrict__ out) {
+    constexpr int D = 128, P = 32, GM = ATT_MAX_G_PF;
+    constexpr bool PAIR = sizeof(KT) == 2;
+    __shared__ float sc[GM][P];
+    __shared__ float qs[GM][D];
+    __shared__ float part[2][GM][D];
+    __shared__ float run_m[GM], run_l[GM], corr_s[GM];
+    const int m = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
+    const int G = nq / nkv, pos = pos0 + m, L = pos + 1;
+    const float* qrow = qkv + (int64_t)m * ldq + (int64_t)g * G * D;
+    // q in the cache's slot order (fp16 rows are paired)
+    for (int e = tid; e < G * D; e += 256) {
+        const int h = e / D, sl = e % D;
+        const int dim = PAIR ? (sl >> 1) + 64 * (sl & 1) : sl;
+        qs[h][sl] = qrow[h * D + dim];
+    }
+    if (tid < GM) {
+        run_m[tid] = -INFINITY;
+        run_l[tid] = 0.f;
+    }
+    const KT* kb = kc + (int64_t)g * max_seq * D;
+    const KT* vb = vc + (int64_t)g * max_seq * D;
+    // output dims of this thread: dims d and d + 64 of heads hh and hh + 2,
+    // over the pass positions of parity ph
+    const int ph = tid >> 7, hh = (tid >> 6) & 1, d = tid & 63;
+    float o0[2] = {0.f, 0.f}, o1[2] = {0.f, 0.f};
+    __syncthreads();
+    const int part8 = tid & 7, sub = tid >> 3;   // 32 positions x 8 slices of 16 slots
+    for (int t0 = 0; t0 < L; t0 += P) {
+        const int np = min(P, L - t0);
+        // the pass's values of this thread's two output dims, loaded with the
+        // keys (positions clamped, used only below np): all in flight at once,
+        // their latency behind the scores (one load round trip per pass; a
+        // load per position in the value loop was one round trip each)
+        float v_lo[P / 2], v_hi[P / 2];
+#pragma unroll
+        for (int jj = 0; jj < P / 2; jj++) {
+            const KT* vr = vb + (int64_t)(t0 + min(ph + 2 * jj, np - 1)) * D;
+            v_lo[jj] = PAIR ? (float)vr[2 * d] : (float)vr[d];
+            v_hi[jj] = PAIR ? (float)vr[2 * d + 1] : (float)vr[d + 64];
+        }
+        {
+            const int t = t0 + sub;
+            float kv[16];
+            const KT* kr = kb + (int64_t)min(t, L - 1) * D + part8 * 16;
+#pragma unroll
+            for (int i = 0; i < 16; i++) kv[i] = (float)kr[i];
+            for (int h = 0; h < G; h++) {
+                float sdot = 0.f;
+#pragma unroll
+                for (int i = 0; i < 16; i++) sdot = fmaf(qs[h][part8 * 16 + i], kv[i], sdot);
+                sdot += __shfl_xor(sdot, 1, 64);
+                sdot += __shfl_xor(sdot, 2, 64);
+                sdot += __shfl_xor(sdot, 4, 64);
+                if (part8 == 0) sc[h][sub] = sub < np ? sdot * scale : -INFINITY;
+            }
+        }
+        __syncthreads();
+        if (tid < 32 * G) {
+            // half-wave h: the pass's max, the running max and sum of head h
+            const int h = tid >> 5, j = tid & 31;
+            const float sv = sc[h][j];
+            float pm = sv;
+#pragma unroll
+            for (int o = 16; o >= 1; o >>= 1) pm = fmaxf(pm, __shfl_xor(pm, o, 64));
+            const float om = run_m[h], nm = fmaxf(om, pm);
+            const float e = j < np ? expf(sv - nm) : 0.f;
+            float es = e;
+#pragma unroll
+            for (int o = 16; o >= 1; o >>= 1) es += __shfl_xor(es, o, 64);
+            sc[h][j] = e;
+            if (j == 0) {
+                const float cr = om == -INFINITY ? 0.f : expf(om - nm);
+                corr_s[h] = cr;
+                run_l[h] = run_l[h] * cr + es;
+                run_m[h] = nm;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int h = hh + 2 * k;
+            if (h < G) {
+                o0[k] *= corr_s[h];
+                o1[k] *= corr_s[h];
+            }
+        }
+#pragma unroll
+        for (int jj = 0; jj < P / 2; jj++) {
+            const int j = ph + 2 * jj;
+            if (j >= np) continue;
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int h = hh + 2 * k;
+                if (h >= G) continue;
+                const float e = sc[h][j];
+                o0[k] = fmaf(e, v_lo[jj], o0[k]);
+                o1[k] = fmaf(e, v_hi[jj], o1[k]);
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int h = hh + 2 * k;
+        if (h < G) {
+            part[ph][h][d] = o0[k];
+            part[ph][h][d + 64] = o1[k];
+        }
+    }
+    __syncthreads();
+    for (int e = tid; e < G * D / 2; e += 256) {
+        const int h = e / (D / 2), dd = 2 * (e % (D / 2));
+        wf_put2(out, m, (g * G + h) * D + dd, nq * D, (part[0][h][dd] + part[1][h][dd]) / run_l[h],
+                (part[0][h][dd + 1] + part[1][h][dd + 1]) / run_l[h]);
+    }
+}
+
 int prefill(Qwen3Dec* d, int M, bool logits) {
     const pio_qwen3_config& c = d->c;
     const int H = c.hidden, D = c.head_dim, nq = c.n_heads, nkv = c.n_kv_heads, I = c.intermediate;
@@ -274,6 +410,7 @@ int prefill(Qwen3Dec* d, int M, bool logits) {
     at.pos0 = pos0;
     at.kv16 = d->kv16;
     at.m_seed = -FLT_MAX;
+    const bool few = pos0 + M <= PF_FEW_KEYS;
     // When a linear's plan splits K, its slices are finished by the next step's
     // own kernel (RoPE + KV rows, SwiGLU, residual + the next RMSNorm) instead
     // of by the GEMM's reduce launch; h_ready: h already holds this layer's
@@ -316,7 +453,18 @@ int prefill(Qwen3Dec* d, int M, bool logits) {
                 at.v = vc;
             }
             PIO_LAUNCHED();
-            PIO_TRY(attn_mfma(at, st));
+            if (few) {
+                const dim3 ag(M, nkv);
+                if (d->kv16)
+                    pf_attn_kernel<_Float16><<<ag, 256, 0, st>>>(qkv, nqkv, pos0, nq, nkv, (const _Float16*)at.k,
+                                                                   (const _Float16*)at.v, c.max_seq, at.scale, o);
+                else
+                    pf_attn_kernel<float><<<ag, 256, 0, st>>>(qkv, nqkv, pos0, nq, nkv, (const float*)at.k,
+                                                                (const float*)at.v, c.max_seq, at.scale, o);
+                PIO_LAUNCHED();
+            } else {
+                PIO_TRY(attn_mfma(at, st));
+            }
         }
         {
             Scratch pw;

@@ -197,6 +197,26 @@ def test_prefill_refuses_generated_positions(torch_dev):
         dec.prefill(1)
 
 
+@pytest.mark.parametrize("kv_dtype", ["float32", "float16"])
+@pytest.mark.parametrize("n_heads", [8, 16, 32])
+def test_prefill_attention_edge(torch_dev, kv_dtype, n_heads):
+    """Either side of the 96 keys up to which a batch's attention has a kernel of
+    its own, with 1, 2 and 4 query heads per KV head: batches of 96, 97 and 60 +
+    37 positions, each against the oracle."""
+    from mod_amd.qwen3 import Qwen3Int8Decoder, random_weights
+    cfg, rcfg = _small(kv_dtype=kv_dtype, n_heads=n_heads)
+    w = random_weights(cfg, seed=71)
+    dec = Qwen3Int8Decoder(cfg, w)
+    prompt = np.random.default_rng(72).integers(0, cfg.vocab, size=97).astype(np.int32)
+    for sizes in ((96,), (97,), (60, 36), (60, 37)):
+        dec.reset(prompt)
+        for n in sizes[:-1]:
+            dec.prefill(n)
+        dec.prefill(sizes[-1], logits=True)
+        got = dec.read(0, with_logits=True)[1]
+        _against_oracle(got[None], prompt, [sum(sizes) - 1], rcfg, w, f"{n_heads} heads, {kv_dtype} KV, batches of {sizes}")
+
+
 @pytest.mark.parametrize("intermediate", [3072, 3088])
 def test_prefill_memory(torch_dev, intermediate):
     """What a batch of 2048 positions takes from the allocator is no more than its
