@@ -25,7 +25,8 @@
 // the end. When there are too few column tiles
 // for the CUs, the keys are split over workgroups as well and a second launch
 // merges the partials. Steps of at most AT_VEC_COLS columns per kv head run on
-// the VALU (attn_vec_kernel).
+// the VALU (attn_vec_kernel). Few rows over few keys have kernels of their own
+// beside the callers (model_ops.hip, prefill.hip).
 //
 // Measured (MI355X; before: a workgroup per query row on the VALU, keys one by
 // one): 777 queries and keys, 16 heads over 8, D 128: 909 -> 72 us; one query

@@ -297,7 +297,7 @@ struct W8pParams {
 // gate rows and the matching up rows, so that a wave holds g and u of the same
 // outputs; silu(g) * u goes through the wave's part of the stages into the
 // planes of act (y), a fragment part per store. It saves the round trip of [g|u]
-// and a launch of 12 us per layer: 0.6B prompt of 1021 positions 6085 -> 5832 us.
+// and a launch of 12 us per layer: 4 % of a 0.6B prompt of 1021 positions.
 template <typename YT, int EPI, int WM, int TN>
 __global__ __launch_bounds__(256, 2) void gemm_w8p_kernel(W8pParams p) {
     constexpr bool SWIGLU = EPI == WF_SWIGLU;

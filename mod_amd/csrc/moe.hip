@@ -423,7 +423,7 @@ static void launch_grouped(const GroupedParams& g, dim3 grid, int nk, hipStream_
 // v_mfma_i32_16x16x64_i8, two sets of MS_SET K values in flight, with the
 // activation rows in LDS; the down kernel quantizes its h rows itself. Same
 // integer sums, scales and order as above, so the same bits.
-// Qwen3-30B-A3B layer: T = 1 36.4 -> 25.2 us. From T = 3 the GEMMs above are the
+// Qwen3-30B-A3B layer: T = 1 37.1 -> 25.6 us. From T = 3 the GEMMs above are the
 // faster ones (41 / 46 us at 3, 86 / 114 at 16): these loads cover half a line of
 // a row each and stream at 4 TB/s, its tiles at 4.6 and up.
 constexpr int MS_MAX_T = 2;        // tokens (and rows of an expert)
