@@ -107,20 +107,19 @@ __device__ __forceinline__ void at_store(const AttnArgs& a, int D, int b, int s,
     }
 }
 
-// A finished column's 4 slots from sl: v, the sum of exp(score - m) v, over l, the
-// sum of the weights; D / 4 consecutive lanes have one column. The sum can leave
-// the fp32 range where softmax(s) v does not (T keys with |v| above FLT_MAX / T),
+// A finished column's 4 slots from sl: r, the sum of exp(score - m) v over l, the
+// sum of the weights; D / 4 consecutive lanes have one column. The first sum can
+// leave the fp32 range where softmax(s) v does not (T keys with |v| above FLT_MAX / T),
 // so a column with an inf or NaN among its outputs whose scores are in order
 // (0 < l < inf) is formed again by its lanes alone, as softmax(s) v is written:
 // the weights' sum, then normalised weights times v, over the keys that the column
 // sees. (In a causal tile an inf or NaN in the value row of a later key meets the
 // zero weights of earlier columns and makes them NaN: they come out right here.)
 template <int D, typename KT, bool CAUSAL>
-__device__ __forceinline__ at_f4 at_finish(const AttnArgs& a, int b, int g, int s, int hd, int sl, at_f4 v, float m,
+__device__ __forceinline__ at_f4 at_finish(const AttnArgs& a, int b, int g, int s, int hd, int sl, at_f4 r, float m,
                                            float l) {
     constexpr bool PAIR = sizeof(KT) == 2;
     constexpr int U = 4;                   // keys at a time
-    const at_f4 r = v / l;
     bool odd = false;
 #pragma unroll
     for (int j = 0; j < 4; j++) odd |= !(fabsf(r[j]) <= FLT_MAX);
@@ -430,7 +429,8 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_mfma_kernel(AttnParams 
             continue;
         }
         const int s = (c0 + c) / p.G, hd = g * p.G + (c0 + c) - s * p.G;
-        at_store<PAIR, CAUSAL>(a, D, b, s, hd, sl, at_finish<D, KT, CAUSAL>(a, b, g, s, hd, sl, v, cm, cl));
+        const at_f4 r = fine ? v / cl : v * (1.0f / cl);   // a rounding less where they are few
+        at_store<PAIR, CAUSAL>(a, D, b, s, hd, sl, at_finish<D, KT, CAUSAL>(a, b, g, s, hd, sl, r, cm, cl));
     }
 }
 
@@ -590,7 +590,7 @@ __global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_vec_kernel(AttnParams p
             }
         } else {
             const int hd = g * p.G + c - s * p.G;
-            at_store<false, false>(a, D, b, s, hd, sl, at_finish<D, float, false>(a, b, g, s, hd, sl, v, cm, cl));
+            at_store<false, false>(a, D, b, s, hd, sl, at_finish<D, float, false>(a, b, g, s, hd, sl, v / cl, cm, cl));
         }
     }
 }
@@ -638,7 +638,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
     }
     const int s = c / p.G, hd = g * p.G + c - s * p.G;
     typedef typename std::conditional<PAIR, _Float16, float>::type KT;
-    at_store<PAIR, CAUSAL>(a, D, b, s, hd, sl, at_finish<D, KT, CAUSAL>(a, b, g, s, hd, sl, v, mx, l));
+    at_store<PAIR, CAUSAL>(a, D, b, s, hd, sl, at_finish<D, KT, CAUSAL>(a, b, g, s, hd, sl, v * (1.0f / l), mx, l));
 }
 
 bool attn_mfma_supported(const AttnArgs& a) {
